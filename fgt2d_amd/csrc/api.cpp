@@ -185,6 +185,11 @@ struct Tables3D {
     double pmax = 0, xmin2 = 0, xm = 0;
     const double *ws = nullptr, *ts = nullptr, *coef = nullptr, *dcoef = nullptr, *wms = nullptr,
                  *wm1 = nullptr;  // wm1: complex (3, npw) m2l factors per axis
+    // shifts of the leaves about their cutoff-level box, per axis: complex
+    // e^{i ts_a off} at (2^d - 1 + place) half + a, a < half, for the 2^d
+    // places of a box d levels below the top one, d = 0..nmax
+    const double* shift = nullptr;
+    bool leafwise = false;  // coef, dcoef and wms are there
 };
 
 // One thread that runs a workspace's host-side job beside the launches of
@@ -546,7 +551,7 @@ Workspace& workspace()
 const char* const kKernels[KID_N] = {"form_moments", "form_h2pw", "form_valu", "merge",
                                      "m2l",          "split",     "pw2local",  "taylor_eval",
                                      "pw_eval",      "direct",    "gather",    "scatter",
-                                     "sort"};
+                                     "sort",         "form_top",  "eval_top"};
 struct KLaunch {
     int id, level;
     double ms;
@@ -896,20 +901,21 @@ const Tables2D& tables2d(Workspace& W, int npw, double pmax, int ntermmax, int n
 // (g3drx2lmat with the i^j grouping), merge/split factors for the 8 octants
 // per shift length (merge_split_pw_matrices, :2760-2842) and the 27 m2l
 // factors (pw_translation_matrices, :2697-2757).  Cached while unchanged.
+// leafwise: the tables of the leaf-by-leaf route (coef, dcoef, wms) as well
 const Tables3D& tables3d(Workspace& W, int npw, double pmax, int ntermmax, int nmax, double xmin2,
-                         double xm, hipStream_t s)
+                         double xm, bool leafwise, hipStream_t s)
 {
     Tables3D& t = W.tab3;
-    if (t.valid && t.npw == npw && t.pmax == pmax && t.ntermmax == ntermmax && t.nmax == nmax &&
+    if (t.valid && (t.leafwise || !leafwise) && t.npw == npw && t.pmax == pmax && t.ntermmax == ntermmax && t.nmax == nmax &&
         t.xmin2 == xmin2 && t.xm == xm)
         return t;
     const int half = npw / 2, mt = ntermmax + 1;
     const size_t nexp = (size_t)npw * npw * half;
     std::vector<double> ws(npw), ts(npw);
     planewave_nodes3(pmax, npw, ws.data(), ts.data());
-    std::vector<double> coef(2 * (size_t)mt * npw), dcoef(2 * (size_t)mt * npw);
+    std::vector<double> coef(leafwise ? 2 * (size_t)mt * npw : 0), dcoef(coef.size());
     double fh = 1.0, fl = 1.0;
-    for (int j = 0; j < mt; ++j) {
+    for (int j = 0; leafwise && j < mt; ++j) {
         if (j > 0) { fh = fh / std::sqrt((double)j); fl = fl * j; }
         for (int a = 0; a < npw; ++a) {
             const double r = ws[a] * std::pow(-ts[a], j) * fh * fh;
@@ -925,8 +931,8 @@ const Tables3D& tables3d(Workspace& W, int npw, double pmax, int ntermmax, int n
         }
     }
     const int nm = std::max(nmax, 1);
-    std::vector<double> wms(2 * nexp * 8 * nm), wm1(2 * 3 * (size_t)npw);
-    {
+    std::vector<double> wms(leafwise ? 2 * nexp * 8 * nm : 0), wm1(2 * 3 * (size_t)npw);
+    if (leafwise) {
         std::vector<double> wr((size_t)npw * (nm + 1)), wi((size_t)npw * (nm + 1));
         for (int j = 0; j < npw; ++j) {
             double zr = std::cos(ts[j] * xmin2), zi = std::sin(ts[j] * xmin2);
@@ -966,9 +972,20 @@ const Tables3D& tables3d(Workspace& W, int npw, double pmax, int ntermmax, int n
         wm1[2 * (3 * j + 1)] = 1;  wm1[2 * (3 * j + 1) + 1] = 0;    // offset 0
         wm1[2 * (3 * j + 2)] = zr; wm1[2 * (3 * j + 2) + 1] = zi;   // offset +1
     }
+    // a box d levels below the top one (size xm, scaled) at place q of 2^d
+    // along an axis is (q + 1/2) xm/2^d - xm/2 off its centre
+    std::vector<double> shift;
+    if (nmax <= TOP_DEPTH)
+        for (int d = 0; d <= nmax; ++d)
+            for (int q = 0; q < (1 << d); ++q)
+                for (int a = 0; a < half; ++a) {
+                    const double off = xm * (2 * q + 1 - (1 << d)) / (double)(2 << d);
+                    shift.push_back(std::cos(ts[a] * off));
+                    shift.push_back(std::sin(ts[a] * off));
+                }
     Pack pk;
     size_t o_ws = pk.add(ws), o_ts = pk.add(ts), o_c = pk.add(coef), o_d = pk.add(dcoef);
-    size_t o_ms = pk.add(wms), o_ml = pk.add(wm1);
+    size_t o_ms = pk.add(wms), o_ml = pk.add(wm1), o_sh = pk.add(shift);
     char* d = W.get<char>("tables3", pk.size());
     HIPCHECK(hipMemcpyAsync(d, pk.data(), pk.size(), hipMemcpyHostToDevice, s));
     HIPCHECK(hipStreamSynchronize(s));  // pk is freed on return
@@ -978,6 +995,8 @@ const Tables3D& tables3d(Workspace& W, int npw, double pmax, int ntermmax, int n
     t.dcoef = (const double*)(d + o_d);
     t.wms = (const double*)(d + o_ms);
     t.wm1 = (const double*)(d + o_ml);
+    t.shift = (const double*)(d + o_sh);
+    t.leafwise = leafwise;
     t.valid = true;
     t.npw = npw;
     t.pmax = pmax;
@@ -2078,6 +2097,68 @@ void run_large_delta3(Workspace& W, const Call& q, hipStream_t s, int npwlevel, 
 // routes chosen by (p+1)/npw and the box's point count (fgt3d.f:971-983,
 // :1297-1310), listpw without leaf colleagues, near field with
 // dmax = ln(1/eps) delta and the 3D modified list1 (tree_routs3d.f:511-620).
+// Route of a 3D transform with expansions: whole cutoff-level boxes at once
+// (k_form3_top, k_eval3_top) or leaf by leaf, whichever the estimate below
+// finds faster; the values are the same but for rounding.  The first costs
+// 2 npw^3 operations a point at every order; the second the conversions and
+// shifts of every leaf, and a few operations a point at the low orders of the
+// finest level, so it keeps the transforms with many points in every leaf.
+// The constants (ns) are fits to both routes over uniform and shell points,
+// 5*10^3 to 4*10^6 of them, delta 1e-4..1e-2, eps 1e-3, 1e-6, 1e-9:
+//   at once    8e-5 npw^3 + 0.2 a source and an evaluated point (with
+//              gradients 2.7, Hessians 7 times, formation with dipoles twice);
+//              a box of sources is one block's serial sum, which bounds the
+//              formation where few boxes hold most of the sources;
+//   by leaves  50 + 8.75e-3 npw^3 a leaf of order <= 16, 50 + 2.5e-2 npw^3 of
+//              order <= 32, 0.44 npw^3 above (kernels without matrix cores),
+//              1.5e-4 m^3 a point and side; 30 us of more launches.
+// Measured (by leaves -> at once): 10^6 points, delta 1e-3, eps 1e-6 (23 a
+// leaf): 11.0 -> 4.8 ms; delta 3e-3 (111 a leaf): 2.8 -> 4.0 ms, so there by
+// leaves; 4*10^5, delta 3e-3, eps 1e-9 (21 a leaf): 22.4 -> 6.1 ms.
+bool top_route3(const std::vector<LeafRun>& leaves, const Call& q, int ltop, int npwlevel,
+                int nlevels, int npw, const std::vector<int>& nlocal)
+{
+    if (nlevels - ltop > TOP_DEPTH || nlevels >= TOP_LEVELS) return false;
+    const double n3 = (double)npw * npw * npw;
+    // sources and leaves below the cutoff level, and the fullest box there
+    double cost[TOP_LEVELS], m3[TOP_LEVELS];
+    size_t count[TOP_LEVELS] = {};
+    for (int l = ltop; l <= nlevels; ++l) {
+        const int m = nlocal[l] + 1;
+        cost[l] = m <= 16 ? 50 + 8.75e-3 * n3 : (m <= 32 ? 50 + 2.5e-2 * n3 : 0.44 * n3);
+        m3[l] = 1.5e-4 * m * m * m;
+    }
+    double leafwise = 3e4, nsum = 0, psum = 0;
+    int most = 0, here = 0;
+    uint64_t last = ~(uint64_t)0;
+    const size_t n = leaves.size();
+    for (size_t i = 0; i < n; ++i) {
+        const int l = leaves[i].level;
+        if (l < ltop || l <= npwlevel) continue;
+        const int c = (i + 1 < n ? leaves[i + 1].start : q.ns) - leaves[i].start;
+        const uint64_t box = leaves[i].key >> (3 * (l - ltop));
+        here = box == last ? here + c : c;
+        last = box;
+        most = std::max(most, here);
+        ++count[l];
+        psum += m3[l] * c;
+        nsum += c;
+    }
+    // fewer leaves than CUs leave the chip idle
+    for (int l = ltop; l <= nlevels; ++l)
+        if (count[l]) leafwise += cost[l] * std::max<size_t>(count[l], 256);
+    auto weight = [](int ifpgh) { return ifpgh <= 0 ? 0.0 : (ifpgh == 1 ? 1.0 : (ifpgh == 2 ? 2.7 : 7.0)); };
+    // evaluated points as if spread like the sources
+    const double es = q.ifpgh > 0 ? 1.0 : 0.0;
+    const double et = q.ifpghtarg > 0 ? (double)q.nt / q.ns : 0.0;
+    const double dip = q.rn ? 2.0 : 1.0;
+    leafwise += psum * (1.0 + es + et);
+    const double pt = 8e-5 * n3 + 0.2;
+    const double form = pt * dip * std::max(nsum, 130.0 * most);
+    const double eval = pt * nsum * (weight(q.ifpgh) + et * weight(q.ifpghtarg));
+    return form + eval < leafwise;  // every density costs the same again
+}
+
 void run3d(Workspace& W, const Call& q, hipStream_t s)
 {
     t_mixed = false;
@@ -2305,6 +2386,9 @@ void run3d(Workspace& W, const Call& q, hipStream_t s)
     std::vector<std::vector<int>> form_l(nlevels + 1), merge_l(nlevels + 1), split_l(nlevels + 1),
         eval_l(nlevels + 1);
     std::vector<int> m2l_l;
+    // the cutoff-level boxes formed and evaluated whole (k_form3_top, k_eval3_top)
+    std::vector<int> tform_l, teval_l;
+    const bool top = expansions && top_route3(leaves, q, nlevstart, npwlevel, nlevels, npw, nlocal);
     // chunks: upward (level of the formed leaves, first and last parent in
     // merge_l[level - 1], first and last leaf in form_l[level]); downward
     // (level, first and last box in eval_l[level])
@@ -2327,7 +2411,21 @@ void run3d(Workspace& W, const Call& q, hipStream_t s)
                     if (T.nch[T.col[27 * b + i]] > 0) { iflocal[b] = 1; break; }
             }
         const int lform = std::max(npwlevel + 1, 0);
-        for (int l = nlevstart; l <= nlevels; ++l)
+        if (top)
+            for (int b = T.laddr[2 * nlevstart]; b <= T.laddr[2 * nlevstart + 1]; ++b) {
+                const bool evaluated =
+                    T.nch[b] > 0 || !(nlevstart == npwlevel && !iflocal[b]);
+                if (T.nch[b] > 0 || nlevstart >= lform) {
+                    tform_l.push_back(b);
+                    slot_mp[b] = n_mp++;
+                }
+                if (evaluated) {
+                    m2l_l.push_back(b);
+                    teval_l.push_back(b);
+                    slot_loc[b] = n_loc++;
+                }
+            }
+        for (int l = nlevstart; l <= (top ? nlevstart - 1 : nlevels); ++l)
             for (int b = T.laddr[2 * l]; b <= T.laddr[2 * l + 1]; ++b) {
                 if (T.nch[b] > 0 && l <= nlevels - 1) {
                     merge_l[l].push_back(b);
@@ -2376,6 +2474,7 @@ void run3d(Workspace& W, const Call& q, hipStream_t s)
         const double G = 1024.0 * 1024.0 * 1024.0;
         const double avail = (double)fr + W.held("exp3") + W.held("taylor3") - 1.0 * G - 0.02 * tot;
         const double pers = 8.0 * per * ((double)n_mp + n_loc);
+        if (top) need_tay = 1, m3max = 1;
         const double full = pers + 8.0 * per * need_c + 8.0 * need_tay;
         size_t cap_c = need_c, cap_tay = need_tay;
         if (full > avail) {
@@ -2459,10 +2558,15 @@ void run3d(Workspace& W, const Call& q, hipStream_t s)
         }
         o_m2l = pk.add(m2l_l);
     }
+    size_t o_lev = 0, o_lofr = 0, o_tform = 0, o_teval = 0;
+    if (top) {
+        o_lev = pk.add(T.lev), o_lofr = pk.add(T.leaf_of_rank);
+        o_tform = pk.add(tform_l), o_teval = pk.add(teval_l);
+    }
     const Tables3D& tab = expansions
                               ? tables3d(W, npw, pmax, ntermmax, nlevels - nlevstart,
                                          T.bsz[nlevels] / std::sqrt(q.delta) / 2,
-                                         T.bsz[nlevstart] / std::sqrt(q.delta), s)
+                                         T.bsz[nlevstart] / std::sqrt(q.delta), !top, s)
                               : W.tab3;
 
     // near field: modified list1 of the source leaves at or above the cutoff
@@ -2598,7 +2702,90 @@ void run3d(Workspace& W, const Call& q, hipStream_t s)
     }
 
     // ---------------- expansions: steps 1-5 ----------------
-    if (expansions) {
+    if (top) {
+        double* mp = W.get<double>("exp3", per * ((size_t)n_mp + n_loc));
+        double* lc = mp + per * (size_t)n_mp;
+        // leaf of every sorted point, in place of arrays that are free by now
+        int* pb_s = lvl;
+        int* pb_t = use_trg ? (int*)W.get<u64>("keys_t", nt) : nullptr;
+        TopRec* rec = W.get<TopRec>("leaf_rec", nleaves);
+        const size_t nte = teval_l.size(), sg_t = nte + nt / 64 + 1, sg_s = nte + ns / 64 + 1;
+        int* seg_t = W.get<int>("tstart", 2 * (nte + 1) + (use_trg ? sg_t : 0) + (use_src ? sg_s : 0));
+        int* seg_s = seg_t + nte + 1;
+        int* box_t = seg_s + nte + 1;
+        int* box_s = box_t + (use_trg ? sg_t : 0);
+        SegLists L{};
+        const int* d_teval = (const int*)D(o_teval);
+        if (use_trg) L.l[L.count++] = SegList{d_teval, (int)nte, trg_se, 64, seg_t, box_t};
+        if (use_src) L.l[L.count++] = SegList{d_teval, (int)nte, src_se, 64, seg_s, box_s};
+        launch_seg_scan(L, s);
+        Top3Args ta{};
+        ta.cen = d_cen;
+        ta.rec = rec;
+        ta.nd = nd;
+        ta.dsq = dsq;
+        ta.npw = npw;
+        ta.ltop = nlevstart;
+        ta.ws = tab.ws;
+        ta.ts = tab.ts;
+        ta.shift = (const double2*)tab.shift;
+        ta.nshift = ((2 << (nlevels - nlevstart)) - 1) * half;
+        for (int l = nlevstart; l <= nlevels; ++l) {
+            ta.m[l] = nlocal[l] + 1;
+            ta.thresh[l] = form_thresh[l];
+            ta.ib[l] = 1.0 / T.bsz[l];
+        }
+        launch_top_leaves(ta, ls, tg ? ls2 : nullptr, nleaves, (const int*)D(o_lofr),
+                          (const int*)D(o_lev), d_par, pb_s, pb_t, rec, s);
+        tm.begin(S_FORM);
+        for (int ind = 0; ind < nd; ++ind) {
+            Top3Args fa = ta;
+            fa.tops = (const int*)D(o_tform);
+            fa.ntop = (int)tform_l.size();
+            fa.se = src_se;
+            fa.pbox = pb_s;
+            fa.pts = xs;
+            fa.qs = qs;
+            fa.dipw = wsd;
+            fa.ind = ind;
+            fa.slot = d_smp;
+            fa.mp = mp;
+            tm.ctx(nlevstart, &tform_l, 0);
+            launch_form3_top(fa, s);
+        }
+        tm.end(S_FORM);
+        tm.begin(S_M2L);
+        tm.ctx(nlevstart, &m2l_l, 2);
+        launch_m2l3((const int*)D(o_m2l), (int)m2l_l.size(), d_cen, d_ncol, d_col, d_nch, src_se,
+                    trg_se, use_src, use_trg, d_smp, d_sloc, tab.wm1, npw, T.bsz[nlevstart],
+                    nlevstart == npwlevel, nd, nexp, mp, lc, s);
+        tm.end(S_M2L);
+        tm.begin(S_EVAL);
+        for (int side = 0; side < 2; ++side) {
+            if (side == 0 ? !use_trg : !use_src) continue;
+            Top3Args ea = ta;
+            ea.tops = d_teval;
+            ea.ntop = (int)teval_l.size();
+            ea.se = side == 0 ? trg_se : src_se;
+            ea.pbox = side == 0 ? pb_t : pb_s;
+            ea.pts = side == 0 ? xt : xs;
+            ea.slot = d_sloc;
+            ea.mp = lc;
+            ea.tstart = side == 0 ? seg_t : seg_s;
+            ea.segbox = side == 0 ? box_t : box_s;
+            ea.grid = (int)std::min<long>(1 << 16, ea.ntop + (side == 0 ? nt : ns) / 64 + 1);
+            ea.ifpgh = side == 0 ? q.ifpghtarg : q.ifpgh;
+            ea.pot = side == 0 ? pt : ps;
+            ea.grad = side == 0 ? gt : gs;
+            ea.hess = side == 0 ? ht : hs;
+            for (int ind = 0; ind < nd; ++ind) {
+                ea.ind = ind;
+                tm.ctx(nlevstart, &teval_l, side == 0 ? 1 : 0);
+                launch_eval3_top(ea, s);
+            }
+        }
+        tm.end(S_EVAL);
+    } else if (expansions) {
         double* xb = W.get<double>("exp3", per * ((size_t)n_mp + n_loc + ncap));
         double* mp = xb;                       // multipole slots
         double* lc = xb + per * (size_t)n_mp;  // local slots (the chunk region follows)

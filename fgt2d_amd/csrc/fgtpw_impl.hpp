@@ -30,7 +30,8 @@ void check_hip(hipError_t e, const char* what);
 // ---------------------------------------------------------------------------
 enum KernelId {
     KID_FORM_MOMENTS, KID_FORM_H2PW, KID_FORM_VALU, KID_MERGE, KID_M2L, KID_SPLIT, KID_PW2LOCAL,
-    KID_TAYLOR_EVAL, KID_PW_EVAL, KID_DIRECT, KID_GATHER, KID_SCATTER, KID_SORT, KID_N
+    KID_TAYLOR_EVAL, KID_PW_EVAL, KID_DIRECT, KID_GATHER, KID_SCATTER, KID_SORT, KID_FORM_TOP,
+    KID_EVAL_TOP, KID_N
 };
 struct KernelClock {
     // events recorded on the stream before (end = false) and after the
@@ -353,6 +354,49 @@ struct Form3Args {
 void launch_form3_hermite(const Form3Args& a, hipStream_t s);
 long form3_mfma_scratch(int m, int npw);  // per-block scratch of the matrix-core route
 void launch_form3_pw(const Form3Args& a, hipStream_t s);
+
+// Formation and evaluation at the cutoff level (k_form3_top, k_eval3_top)
+constexpr int TOP_LEVELS = 24, TOP_DEPTH = 4;  // levels; of these below the cutoff level
+struct TopRec {             // one leaf, as the phase tables need it
+    double c[3];            // centre
+    int row[3];             // shift table rows per axis (offset of node 0)
+    int mf, me;             // terms of its series, formation and evaluation; -1: whole exponentials
+};
+struct Top3Args {
+    const int* tops;        // cutoff-level boxes
+    int ntop;
+    const double* cen;      // 3 per box
+    const int2* se;         // point ranges of the boxes (sources, or the evaluated points)
+    const int* pbox;        // leaf rank of every sorted point
+    const TopRec* rec;      // per leaf rank
+    const double* pts;      // sorted points (3,n)
+    const double* qs;       // formation: sorted charges (nd,n)
+    const double* dipw;     // formation: dipole weights d n, (n, nd, 3) sorted, or nullptr
+    int nd, ind;
+    double dsq;
+    int npw, ltop;
+    const double *ws, *ts;  // nodes (ascending)
+    const double2* shift;   // e^{i ts_a (c_leaf - c_top)}, a < npw/2: rows 2^d - 1 + place
+    int nshift;             // along the axis, d levels below the top; entries of the table
+    const int* slot;
+    double* mp;             // per slot (nd, nexp) complex: written, or read by the evaluation
+    // per level: terms of the leaves' series, route threshold (as Form3Args,
+    // Eval3Args), 1 / box size
+    int m[TOP_LEVELS], thresh[TOP_LEVELS];
+    double ib[TOP_LEVELS];
+    // evaluation: segments of 64 points (tstart, segbox as SegList), outputs
+    // accumulated
+    const int *tstart, *segbox;
+    int grid, ifpgh;
+    double *pot, *grad, *hess;
+};
+void launch_form3_top(const Top3Args& a, hipStream_t s);
+void launch_eval3_top(const Top3Args& a, hipStream_t s);
+// pb[i] = r for the sources ls[r] <= i < ls[r + 1] of every leaf rank (pb2:
+// the targets of ls2, or nullptr), and the leaves' records
+void launch_top_leaves(const Top3Args& a, const int* ls, const int* ls2, int nleaves,
+                       const int* leaf_of_rank, const int* lev, const int* par, int* pb, int* pb2,
+                       TopRec* rec, hipStream_t s);
 
 void launch_merge3(const int* parents, int np, const int* child8, const double* cen,
                    const int2* src_se, const int* slot, const double* wms, int kbase, int nd,

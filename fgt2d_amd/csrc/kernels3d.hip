@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <mutex>
 
 #include "fgtpw_impl.hpp"
@@ -2075,6 +2076,746 @@ void launch_pw_eval3(const Eval3Args& a, hipStream_t s)
     else
         k_pw_eval3<1><<<a.grid, 256, 0, s>>>(a);
     kmark(KID_PW_EVAL, true, s);
+}
+
+// ---------------------------------------------------------------------------
+// Steps 1-2 and 4-5 at the cutoff level, for every point of a cutoff-level
+// box at once.  The Hermite / Taylor route of a leaf truncates each axis'
+// exponential after m terms about the leaf's centre; that polynomial, moved
+// to the cutoff-level ancestor's centre, is the real pair
+//   (C + iS)(x, a) = [sum_{j<m} (i ts_a u)^j / j!] e^{i ts_a (c_leaf - c_top)},
+// u = (x - c_leaf)/sqrt(delta) -- or e^{i ts_a u} whole, where the leaf is on
+// the plane-wave route.  The formation (with its merges) and the evaluation
+// (with its splits) of the box are then one real product each over its points:
+//   mp(a,b,c)  = sum_s q (C-iS)(x,a) (C-iS)(y,b) (C-iS)(z,c) ws_a ws_b ws_c
+//   pot(p)     = 2 Re sum (C+iS)(x,a) (C+iS)(y,b) (C+iS)(z,c) loc(a,b,c).
+// Mirror nodes are conjugates, so the cosines and sines of the first half of
+// an axis' nodes span it: npw real rows and columns, 2 npw^3 operations a
+// point, on FP64 matrix cores.  No leaf expansion is formed, stored, merged,
+// split or converted; the values differ from the leaf-by-leaf route by
+// rounding alone (2-norm 1e-15).
+// Bound by the FP64 matrix pipe (64 cycles an MFMA, about 40% busy), behind
+// it the phase tables and barriers.  Against the leaf kernels they replace,
+// us: 10^6 uniform points, eps 1e-6 (npw 26): formation and merge 4500 ->
+// 1420, conversion, split and evaluation 4270 -> 1420; 8M shell sources + 8M
+// targets, eps 1e-9 (npw 38): 126000 -> 34000 and 158000 -> 15000; 5*10^4
+// sources with gradients, 2*10^4 targets with Hessians (npw 44, leaves of
+// order 34): 5690 -> 380 and 20700 -> 1930.
+// ---------------------------------------------------------------------------
+constexpr int TOP_RF = 66;  // 1/j!, j < TOP_RF
+struct TopFactorials {
+    double v[TOP_RF];
+    constexpr TopFactorials() : v()
+    {
+        double f = 1.0;
+        for (int j = 0; j < TOP_RF; ++j) {
+            if (j > 0) f *= j;
+            v[j] = 1.0 / f;
+        }
+    }
+};
+__constant__ const TopFactorials c_rf = TopFactorials();
+
+// one point alone; not inlined: the rare path must not cost the common one
+// its registers
+__device__ __noinline__ double2 top_series1(double u, int m)
+{
+    double c = 0, sn = 0;
+    if (m < 0) {
+        sincos(u, &sn, &c);
+        return make_double2(c, sn);
+    }
+    const double v = -u * u;
+    int k = (m - 1) >> 1;  // cosine terms 0..k, sine terms 0..k (k - 1 for odd m)
+    if (m & 1) {
+        c = c_rf.v[2 * k];
+        --k;
+    }
+    for (; k >= 0; --k) {
+        c = c * v + c_rf.v[2 * k];
+        sn = sn * v + c_rf.v[2 * k + 1];
+    }
+    return make_double2(c, sn * u);
+}
+
+// e[i] = sum_{j<m[i]} (i u[i])^j / j!; m[i] < 0: e^{i u[i]}.  U independent
+// Horner chains at once; where every m of the wavefront is the same (points of
+// one level) the factorials are scalar loads.
+template <int U>
+__device__ __forceinline__ void top_series(const double (&u)[U], const int (&m)[U], double2 (&e)[U])
+{
+    const int mu = __builtin_amdgcn_readfirstlane(m[0]);
+    bool same = true;
+#pragma unroll
+    for (int i = 0; i < U; ++i) same = same && m[i] == mu;
+    if (__all(same) && mu >= 0) {
+        double v[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+            v[i] = -u[i] * u[i];
+            e[i] = make_double2(0.0, 0.0);
+        }
+        int k = (mu - 1) >> 1;
+        if (mu & 1) {
+#pragma unroll
+            for (int i = 0; i < U; ++i) e[i].x = c_rf.v[2 * k];
+            --k;
+        }
+        for (; k >= 0; --k) {
+            const double fc = c_rf.v[2 * k], fs = c_rf.v[2 * k + 1];
+#pragma unroll
+            for (int i = 0; i < U; ++i) {
+                e[i].x = e[i].x * v[i] + fc;
+                e[i].y = e[i].y * v[i] + fs;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i) e[i].y *= u[i];
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < U; ++i) e[i] = top_series1(u[i], m[i]);
+}
+
+// a point's leaf as the phase tables need it
+struct TopLeaf {
+    double u[3];  // (x - c_leaf)/sqrt(delta)
+    int row[3];   // shift table rows (offset of node 0)
+    int m;        // terms; -1: whole exponentials
+};
+
+__device__ __forceinline__ TopLeaf top_leaf(const Top3Args& a, long i, bool form)
+{
+    TopLeaf L;
+    const TopRec q = a.rec[a.pbox[i]];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        L.u[k] = (a.pts[3 * i + k] - q.c[k]) * a.dsq;
+        L.row[k] = q.row[k];
+    }
+    L.m = form ? q.mf : q.me;
+    return L;
+}
+
+// e times the shift
+__device__ __forceinline__ double2 top_shift(const double2 e, const double2 sh)
+{
+    return make_double2(e.x * sh.x - e.y * sh.y, e.x * sh.y + e.y * sh.x);
+}
+// m - k terms (the k-th derivative's), whole exponentials staying whole
+__device__ __forceinline__ int top_less(int m, int k) { return m < 0 ? m : max(m - k, 0); }
+
+// Formation.  One block of 4 wavefronts per (box, run of 4 TW column tiles):
+// rows (cos, sin) of the x nodes, columns (y node, z node, cos or sin of y, re
+// or im of z and the charge) packed without padding between z nodes, sources
+// as the MFMA K dimension.  Row order: a 16-row tile holds 8 nodes, cosine and
+// sine of a node in neighbouring result registers of one lane; the four
+// columns of a (y, z) pair sit in neighbouring lanes, which between them write
+// the four mirror images of (a, b).  The tables of a chunk of sources are
+// built by all lanes, four sources at a time in each; two blocks per CU
+// overlap one's tables with the other's products.
+// With dipoles the products are X [Y (q Z + w3 Z') + Y' w2 Z] + X' [Y w1 Z],
+// primes the derivatives along the axis.
+template <int NB>
+constexpr int FORM_TW = NB == 1 ? 8 : (NB == 2 ? 4 : (NB == 3 ? 6 : 8));  // column tiles of a wavefront
+constexpr int FORM_ZC = 12;  // z nodes a block's columns reach at most
+
+template <int NB, bool DIP>
+__global__ __launch_bounds__(256, NB <= 3 ? 2 : 1) void k_form3_top(Top3Args a)
+{
+    constexpr int S = 16 * (NB | 1);       // row stride of the tables (odd multiple of 16)
+    constexpr int NS = DIP || NB > 3 ? 32 : 64;  // sources per chunk
+    constexpr int NZ = DIP ? 3 : 1, ZS = 2 * NZ * FORM_ZC, TW = FORM_TW<NB>;
+    extern __shared__ double sm[];
+    double* X = sm;                         // [NS][S]
+    double* Y = X + NS * S;
+    double* X1 = DIP ? Y + NS * S : Y;
+    double* Y1 = DIP ? X1 + NS * S : Y;
+    double* Z = Y1 + NS * S;                // complex [NS][z nodes][NZ]
+    double* rec = Z + NS * ZS;              // per source: u (3), q, w (3), unused
+    int* irec = (int*)(rec + 8 * NS);       // rows (3), m
+    double2* shl = (double2*)(irec + 4 * NS);  // the shift table
+    const int t = threadIdx.x, w = t >> 6, lane = t & 63, i16 = lane & 15, k4 = lane >> 4;
+    const int npw = a.npw, half = npw / 2;
+    const int ncol = npw * npw, ntile = (ncol + 15) / 16, nrun = (ntile + 4 * TW - 1) / (4 * TW);
+    const int run = blockIdx.x % nrun, box = a.tops[blockIdx.x / nrun];
+    // this run's tiles, spread evenly; wavefront w takes every 4th
+    const int tb = (int)((long)ntile * run / nrun), te = (int)((long)ntile * (run + 1) / nrun);
+    const int c0 = 4 * tb / half;           // first z node: 16 tb / (4 half)
+    const int c1 = min(half, (4 * te - 1) / half + 1);
+    const long nexp = (long)npw * npw * half;
+    const int2 r = a.se[box];
+    for (int o = t; o < (DIP ? 4 : 2) * NS * S; o += 256) X[o] = 0.0;  // padding stays zero
+    for (int o = t; o < NS * ZS; o += 256) Z[o] = 0.0;
+    // this lane's column of every tile: y table place, z table place
+    int yo[TW], zo[TW];
+#pragma unroll
+    for (int i = 0; i < TW; ++i) {
+        const int col = 16 * (tb + w + 4 * i) + i16, bc = col >> 2;
+        const bool in = col < ncol && tb + w + 4 * i < te;
+        const int c = in ? bc / half : c0, b = in ? bc % half : 0;
+        yo[i] = 2 * b + ((col >> 1) & 1);
+        zo[i] = 2 * NZ * (c - c0) + (col & 1);
+    }
+    // lanes over the items of a source (x nodes, y nodes, z nodes), two
+    // sources per wavefront where they fit
+    const int items = 2 * half + c1 - c0, span = items <= 32 ? 32 : 64;
+    const int lsrc = w * (64 / span) + (span == 32 ? lane >> 5 : 0), nsrc = 4 * (64 / span);
+    d4_t3 acc[NB][TW];
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < TW; ++j) acc[i][j] = (d4_t3){0, 0, 0, 0};
+    for (int o = t; o < a.nshift; o += 256) shl[o] = a.shift[o];
+    // the next chunk's points and their leaves are loaded beside the products
+    // (the barriers order LDS only); past the end: the last source's place, no
+    // charge or strength
+    double px[3], pq = 0, pd[3] = {0, 0, 0};
+    TopRec pr;
+    int pb = 0;
+    auto leaf = [&](int s0) { return min(s0 + t, r.y - 1); };
+    auto fetch = [&](int s0) {
+        const long i = leaf(s0);
+        const bool in = s0 + t < r.y;
+        const long o = (long)a.nd * i + a.ind;
+        pr = a.rec[pb];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) px[k] = a.pts[3 * i + k];
+        pq = in ? a.qs[o] : 0.0;
+        if (DIP)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) pd[k] = in ? a.dipw[3 * o + k] : 0.0;
+        pb = a.pbox[leaf(s0 + NS)];
+    };
+    if (t < NS && r.x < r.y) {
+        pb = a.pbox[leaf(r.x)];
+        fetch(r.x);
+    }
+    for (int s0 = r.x; s0 < r.y; s0 += NS) {
+        const int cn = min(NS, r.y - s0);
+        if (t < NS) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                rec[8 * t + k] = (px[k] - pr.c[k]) * a.dsq;
+                irec[4 * t + k] = pr.row[k];
+                if (DIP) rec[8 * t + 4 + k] = a.dsq * pd[k];
+            }
+            irec[4 * t + 3] = pr.mf;
+            rec[8 * t + 3] = pq;
+        }
+        lds_barrier3();  // and the last chunk's products are done
+        const int nks = (cn + 3) / 4;
+        for (int f = lane & (span - 1); f < items; f += span) {
+            const int ax = f < half ? 0 : (f < 2 * half ? 1 : 2);
+            const int node = ax == 0 ? f : (ax == 1 ? f - half : c0 + f - 2 * half);
+            const double tsn = a.ts[node], wsn = a.ws[node];
+            constexpr int U = 4;
+            for (int sl0 = lsrc; sl0 < 4 * nks; sl0 += U * nsrc) {
+                double u[U];
+                int m[U];
+                double2 sh[U], e[U], e1[U];
+#pragma unroll
+                for (int i = 0; i < U; ++i) {
+                    const int sl = sl0 + i * nsrc;
+                    u[i] = tsn * rec[8 * sl + ax];
+                    m[i] = irec[4 * sl + 3];
+                    sh[i] = shl[irec[4 * sl + ax] + node];
+                }
+                top_series<U>(u, m, e);
+                if (DIP) {
+                    // (C', S') = ts (-S, C) of one term fewer
+#pragma unroll
+                    for (int i = 0; i < U; ++i) m[i] = top_less(m[i], 1);
+                    top_series<U>(u, m, e1);
+                }
+#pragma unroll
+                for (int i = 0; i < U; ++i) {
+                    const int sl = sl0 + i * nsrc;
+                    e[i] = top_shift(e[i], sh[i]);
+                    e[i].x *= wsn;
+                    e[i].y *= wsn;
+                    if (DIP) {
+                        const double2 g = top_shift(e1[i], sh[i]);
+                        e1[i] = make_double2(-tsn * wsn * g.y, tsn * wsn * g.x);
+                    }
+                    if (ax == 0) {
+                        double* p = X + sl * S + 16 * (node >> 3) + (node & 3) + 8 * ((node >> 2) & 1);
+                        p[0] = e[i].x;
+                        p[4] = e[i].y;
+                        if (DIP) {
+                            p[X1 - X] = e1[i].x;
+                            p[X1 - X + 4] = e1[i].y;
+                        }
+                    } else if (ax == 1) {
+                        *(double2*)(Y + sl * S + 2 * node) = e[i];
+                        if (DIP) *(double2*)(Y1 + sl * S + 2 * node) = e1[i];
+                    } else {
+                        // Z = C - iS
+                        double* p = Z + sl * ZS + 2 * NZ * (node - c0);
+                        const double q = rec[8 * sl + 3];
+                        if (!DIP) {
+                            *(double2*)p = make_double2(q * e[i].x, -q * e[i].y);
+                        } else {
+                            const double w1 = rec[8 * sl + 4], w2 = rec[8 * sl + 5],
+                                         w3 = rec[8 * sl + 6];
+                            *(double2*)p = make_double2(q * e[i].x + w3 * e1[i].x,
+                                                        -(q * e[i].y + w3 * e1[i].y));
+                            *(double2*)(p + 2) = make_double2(w2 * e[i].x, -w2 * e[i].y);
+                            *(double2*)(p + 4) = make_double2(w1 * e[i].x, -w1 * e[i].y);
+                        }
+                    }
+                }
+            }
+        }
+        if (t < NS && s0 + NS < r.y) fetch(s0 + NS);
+        lds_barrier3();
+        for (int ks = 0; ks < nks; ++ks) {
+            const int sa = 4 * ks + k4;
+            double xa[NB], xb[NB];
+#pragma unroll
+            for (int mt = 0; mt < NB; ++mt) {
+                xa[mt] = X[sa * S + 16 * mt + i16];
+                xb[mt] = DIP ? X1[sa * S + 16 * mt + i16] : 0.0;
+            }
+#pragma unroll
+            for (int i = 0; i < TW; ++i) {
+                if (tb + w + 4 * i >= te) break;
+                const double y = Y[sa * S + yo[i]];
+                const double* z = Z + sa * ZS + zo[i];
+                double b = y * z[0];
+                if (DIP) b += Y1[sa * S + yo[i]] * z[2 % (2 * NZ)];
+#pragma unroll
+                for (int mt = 0; mt < NB; ++mt) acc[mt][i] = mfma3(xa[mt], b, acc[mt][i]);
+                if (DIP) {
+                    const double gb = y * z[4 % (2 * NZ)];
+#pragma unroll
+                    for (int mt = 0; mt < NB; ++mt) acc[mt][i] = mfma3(xb[mt], gb, acc[mt][i]);
+                }
+            }
+        }
+    }
+    double* out = a.mp + 2 * ((long)a.slot[box] * a.nd + a.ind) * nexp;
+    // lane q = i16 % 4 writes (a, b), (mirror a, b), (a, mirror b), (both)
+    const int l0 = lane & ~3;
+    const double sx = (lane & 1) ? -1.0 : 1.0, sy = (lane & 2) ? -1.0 : 1.0;
+#pragma unroll
+    for (int i = 0; i < TW; ++i) {
+        if (tb + w + 4 * i >= te) break;
+        const int bc = (16 * (tb + w + 4 * i) + i16) >> 2, c = bc / half, b = bc % half;
+        const int bb = (lane & 2) ? npw - 1 - b : b;
+#pragma unroll
+        for (int mt = 0; mt < NB; ++mt)
+#pragma unroll
+            for (int rp = 0; rp < 2; ++rp) {
+                double cv[4], sv[4];  // cos x and sin x rows of the columns cos y re, im, sin y re, im
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    cv[q] = __shfl(acc[mt][i][2 * rp], l0 + q, 64);
+                    sv[q] = __shfl(acc[mt][i][2 * rp + 1], l0 + q, 64);
+                }
+                const int aa = 8 * mt + k4 + 4 * rp, ab = (lane & 1) ? npw - 1 - aa : aa;
+                if (aa >= half || c >= half) continue;
+                // (Cx - i sx Sx)(Cy - i sy Sy) Z
+                *(double2*)(out + 2 * (ab + (long)npw * (bb + (long)npw * c))) =
+                    make_double2(cv[0] - sx * sy * sv[2] + (sx * sv[1] + sy * cv[3]),
+                                 cv[1] - sx * sy * sv[3] - (sx * sv[0] + sy * cv[2]));
+            }
+    }
+}
+
+template <int NB, bool DIP>
+static void form3_top_launch(const Top3Args& a, hipStream_t s)
+{
+    constexpr int S = 16 * (NB | 1), NS = DIP || NB > 3 ? 32 : 64, NZ = DIP ? 3 : 1;
+    constexpr int TW = FORM_TW<NB>;
+    const size_t lds = ((size_t)(DIP ? 4 : 2) * NS * S + (size_t)NS * 2 * NZ * FORM_ZC + 8 * NS) *
+                           sizeof(double) + 4 * NS * sizeof(int) + a.nshift * sizeof(double2);
+    const int ntile = (a.npw * a.npw + 15) / 16, nrun = (ntile + 4 * TW - 1) / (4 * TW);
+    // z nodes of a run's 64 TW columns, 2 npw columns a node
+    if ((64 * TW + 2 * a.npw - 2) / (2 * a.npw) + 1 > FORM_ZC) {
+        // short expansions: one run covers them whole
+        if (a.npw / 2 > FORM_ZC) fail(-3, "formation columns reach too many z nodes");
+    }
+    allow_lds3(k_form3_top<NB, DIP>, lds);
+    klaunch(KID_FORM_TOP, k_form3_top<NB, DIP>, dim3((unsigned)a.ntop * nrun), dim3(256),
+            (unsigned)lds, s, a);
+}
+
+void launch_form3_top(const Top3Args& a, hipStream_t s)
+{
+    if (a.ntop <= 0) return;
+    const int nb = (a.npw + 15) / 16;
+    if (a.npw < 2 || nb > 4) fail(-3, "3D plane-wave length above 64");
+    const bool dip = a.dipw != nullptr;
+    switch (nb) {
+    case 1: dip ? form3_top_launch<1, true>(a, s) : form3_top_launch<1, false>(a, s); break;
+    case 2: dip ? form3_top_launch<2, true>(a, s) : form3_top_launch<2, false>(a, s); break;
+    case 3: dip ? form3_top_launch<3, true>(a, s) : form3_top_launch<3, false>(a, s); break;
+    default: dip ? form3_top_launch<4, true>(a, s) : form3_top_launch<4, false>(a, s); break;
+    }
+}
+
+// Evaluation.  One block of 4 wavefronts per segment of 64 points of one box:
+// a wavefront per 16 points, or where the segment has fewer, two or four
+// wavefronts per 16 points, each with its share of the 16-column tiles.  Per
+// z node c the slab loc(., ., c) is staged as the real matrices
+//   R(k, col), I(k, col): U_c(p) = sum_{k,col} X(p, k) (R + iI)(k, col) Y(p, col),
+// rows k = (x node, cos or sin), columns (y node, cos or sin), from the sums
+// and differences over the mirror nodes; then X R and X I on matrix cores and
+// A(p, col) += z_cos X R - z_sin X I in registers.  The y weights come once,
+// after the last z node: y derivatives cost nothing there, x derivatives take
+// rows of their own, z derivatives accumulators of their own.  Two slab
+// buffers: node c + 1 is loaded into registers before node c is multiplied
+// and written to the other buffer after it, one barrier per node.
+template <int NB, int PGH>
+__global__ __launch_bounds__(256, PGH == 1 && NB <= 2 ? 3 : (PGH < 3 && NB <= 3 ? 2 : 1)) void k_eval3_top(Top3Args a)
+{
+    constexpr int KS = 4 * NB, CS = 16 * NB + 1;
+    constexpr int NP = (64 * NB * NB + 255) / 256;  // (a, b) pairs a thread stages per node
+    constexpr int NX = PGH;              // x rows: values, 1st, 2nd derivatives
+    constexpr int NA = PGH == 1 ? 1 : (PGH == 2 ? 3 : 6);   // (x, z) derivative pairs
+    constexpr int NO = PGH == 1 ? 1 : (PGH == 2 ? 4 : 10);  // outputs
+    extern __shared__ double sm[];
+    const int t = threadIdx.x, w = t >> 6, lane = t & 63, i16 = lane & 15, k4 = lane >> 4;
+    const int npw = a.npw, half = npw / 2, nks = (npw + 3) / 4;
+    const long nexp = (long)npw * npw * half;
+    double* red = sm;                            // [4 wavefronts][NO][16]
+    double* slab = red + 4 * NO * 16;            // 2 x (4 nks rows) x CS of (R, I)
+    const int sstride = 2 * 4 * nks * CS;
+    for (int o = t; o < 2 * sstride; o += 256) slab[o] = 0.0;  // padding stays zero
+    int pa[NP], pb[NP];  // this thread's (a, b) pairs of a slab
+#pragma unroll
+    for (int it = 0; it < NP; ++it) {
+        pa[it] = (t + 256 * it) % half;
+        pb[it] = (t + 256 * it) / half;
+    }
+    const int total = a.tstart[a.ntop];
+    // consecutive blocks go to the 8 dies in turn: each die takes a run of
+    // consecutive segments, whose boxes' slabs then stay in its L2
+    const int run = (total + 7) / 8;
+    for (int vb = blockIdx.x; (vb >> 3) < run; vb += gridDim.x) {
+        const int g = (vb & 7) * run + (vb >> 3);
+        if (g >= total) continue;
+        const int lo = a.segbox[g], box = a.tops[lo];
+        const int2 rr = a.se[box];
+        const int p0 = rr.x + (g - a.tstart[lo]) * 64, p1 = min(rr.y, p0 + 64);
+        const double2* pw = (const double2*)a.mp + ((long)a.slot[box] * a.nd + a.ind) * nexp;
+        // wavefronts per 16 points (1, 2 or 4), this one's points and share
+        const int wl = p1 - p0 > 32 ? 0 : (p1 - p0 > 16 ? 1 : 2), wpt = 1 << wl;
+        const int t0 = p0 + 16 * (w >> wl), sub = w & (wpt - 1);
+        const bool act = t0 < p1 && sub < NB;
+        double2 v[NP][4];
+        auto load = [&](int c) {
+            const double2* pc = pw + (long)npw * npw * c;
+#pragma unroll
+            for (int it = 0; it < NP; ++it)
+                if (pb[it] < half) {
+                    const int aa = pa[it], b = pb[it], am = npw - 1 - aa, bm = npw - 1 - b;
+                    v[it][0] = pc[aa + npw * b];
+                    v[it][1] = pc[am + npw * b];
+                    v[it][2] = pc[aa + npw * bm];
+                    v[it][3] = pc[am + npw * bm];
+                }
+        };
+        auto stage = [&](double* sl) {
+#pragma unroll
+            for (int it = 0; it < NP; ++it) {
+                if (pb[it] < half) {
+                    const int aa = pa[it], b = pb[it];
+                    // sums (S) and differences (D) along x, then along y
+                    const double sxr = v[it][0].x + v[it][1].x, sxi = v[it][0].y + v[it][1].y;
+                    const double dxr = v[it][0].x - v[it][1].x, dxi = v[it][0].y - v[it][1].y;
+                    const double sxr1 = v[it][2].x + v[it][3].x, sxi1 = v[it][2].y + v[it][3].y;
+                    const double dxr1 = v[it][2].x - v[it][3].x, dxi1 = v[it][2].y - v[it][3].y;
+                    double2* q = (double2*)sl + (2 * aa) * CS + 2 * b;
+                    // cos x: S, sin x: iD; sin y: i times the difference
+                    q[0] = make_double2(sxr + sxr1, sxi + sxi1);
+                    q[1] = make_double2(-(sxi - sxi1), sxr - sxr1);
+                    q[CS] = make_double2(-(dxi + dxi1), dxr + dxr1);
+                    q[CS + 1] = make_double2(-(dxr - dxr1), -(dxi - dxi1));
+                }
+            }
+        };
+        load(0);
+        double X[NX][KS], acc[NA][NB][4];
+        const TopLeaf L = top_leaf(a, min(t0 + i16, p1 - 1), false);
+#pragma unroll
+        for (int k0 = 0; k0 < KS; k0 += 4) {
+            double u[4], tsk[4];
+            int m[4];
+            double2 sh[4], e[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int node = min((4 * (k0 + q) + k4) >> 1, half - 1);
+                tsk[q] = a.ts[node];
+                sh[q] = a.shift[L.row[0] + node];
+                u[q] = tsk[q] * L.u[0];
+            }
+#pragma unroll
+            for (int d = 0; d < NX; ++d) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) m[q] = top_less(L.m, d);
+                top_series<4>(u, m, e);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const double2 f = top_shift(e[q], sh[q]);
+                    const bool sn = k4 & 1;
+                    const double x = d == 0 ? (sn ? f.y : f.x)
+                                            : (d == 1 ? tsk[q] * (sn ? f.x : -f.y)
+                                                      : -tsk[q] * tsk[q] * (sn ? f.y : f.x));
+                    X[d][k0 + q] = 4 * (k0 + q) + k4 < npw ? x : 0.0;
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);  // bounds the registers in flight
+        }
+#pragma unroll
+        for (int k = 0; k < NA; ++k)
+#pragma unroll
+            for (int nt = 0; nt < NB; ++nt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[k][nt][r] = 0;
+        __syncthreads();  // the zeros; the last segment's readers are done
+        stage(slab);
+        __syncthreads();
+        for (int c = 0; c < half; ++c) {
+            if (c + 1 < half) load(c + 1);
+            if (act) {
+                // z factors: lane (point i16, derivative k4), fetched per row
+                double vc, vs;
+                {
+                    const double tsn = a.ts[c];
+                    const int dz = PGH == 1 ? 0 : min(k4, PGH - 1);
+                    const double u[1] = {tsn * L.u[2]};
+                    const int m[1] = {top_less(L.m, dz)};
+                    double2 e1[1];
+                    top_series<1>(u, m, e1);
+                    const double2 e = top_shift(e1[0], a.shift[L.row[2] + c]);
+                    vc = dz == 0 ? e.x : (dz == 1 ? -tsn * e.y : -tsn * tsn * e.x);
+                    vs = dz == 0 ? e.y : (dz == 1 ? tsn * e.x : -tsn * tsn * e.y);
+                }
+                const double2* sl = (const double2*)(slab + (c & 1) * sstride) + k4 * CS + i16;
+#pragma unroll
+                for (int nt = 0; nt < NB; ++nt) {
+                    if ((nt & (wpt - 1)) != sub) continue;
+                    d4_t3 T[NX][2];
+#pragma unroll
+                    for (int ix = 0; ix < NX; ++ix) T[ix][0] = T[ix][1] = (d4_t3){0, 0, 0, 0};
+#pragma unroll
+                    for (int ks = 0; ks < KS; ++ks) {
+                        if (ks >= nks) break;
+                        const double2 b = sl[4 * ks * CS + 16 * nt];
+#pragma unroll
+                        for (int ix = 0; ix < NX; ++ix) {
+                            T[ix][0] = mfma3(X[ix][ks], b.x, T[ix][0]);
+                            T[ix][1] = mfma3(X[ix][ks], b.y, T[ix][1]);
+                        }
+                        if ((ks & 3) == 3) __builtin_amdgcn_sched_barrier(0);  // bounds the loads in flight
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        double zc[PGH], zs[PGH];
+#pragma unroll
+                        for (int d = 0; d < PGH; ++d) {
+                            zc[d] = __shfl(vc, k4 + 4 * r + 16 * d, 64);
+                            zs[d] = __shfl(vs, k4 + 4 * r + 16 * d, 64);
+                        }
+                        acc[0][nt][r] += zc[0] * T[0][0][r] - zs[0] * T[0][1][r];
+                        if (PGH >= 2) {
+                            acc[1 % NA][nt][r] += zc[0] * T[1 % NX][0][r] - zs[0] * T[1 % NX][1][r];
+                            acc[2 % NA][nt][r] += zc[1 % PGH] * T[0][0][r] - zs[1 % PGH] * T[0][1][r];
+                        }
+                        if (PGH >= 3) {
+                            acc[3 % NA][nt][r] += zc[0] * T[2 % NX][0][r] - zs[0] * T[2 % NX][1][r];
+                            acc[4 % NA][nt][r] += zc[1 % PGH] * T[1 % NX][0][r] -
+                                                  zs[1 % PGH] * T[1 % NX][1][r];
+                            acc[5 % NA][nt][r] += zc[2 % PGH] * T[0][0][r] - zs[2 % PGH] * T[0][1][r];
+                        }
+                    }
+                }
+            }
+            if (c + 1 < half) stage(slab + ((c + 1) & 1) * sstride);
+            __syncthreads();
+        }
+        // y weights of the rows' points, then the sum over the columns:
+        // pot; gx gy gz; hxx hyy hzz hxy hxz hyz
+        double out[NO][4];
+#pragma unroll
+        for (int k = 0; k < NO; ++k)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) out[k][r] = 0;
+#pragma unroll
+        for (int nt = 0; nt < NB; ++nt) {
+            if ((nt & (wpt - 1)) != sub) continue;
+            const int col = 16 * nt + i16, node = min(col >> 1, half - 1);
+            const double tsn = a.ts[node];
+            double u[4], y[PGH][4];
+            int m0[4], m[4];
+            double2 sh[4], e[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                u[r] = tsn * __shfl(L.u[1], k4 + 4 * r, 64);
+                sh[r] = a.shift[__shfl(L.row[1], k4 + 4 * r, 64) + node];
+                m0[r] = __shfl(L.m, k4 + 4 * r, 64);
+            }
+#pragma unroll
+            for (int d = 0; d < PGH; ++d) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) m[r] = top_less(m0[r], d);
+                top_series<4>(u, m, e);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const double2 f = top_shift(e[r], sh[r]);
+                    const bool sn = col & 1;
+                    y[d][r] = col < npw ? (d == 0 ? (sn ? f.y : f.x)
+                                                  : (d == 1 ? tsn * (sn ? f.x : -f.y)
+                                                            : -tsn * tsn * (sn ? f.y : f.x)))
+                                        : 0.0;
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                out[0][r] += y[0][r] * acc[0][nt][r];
+                if (PGH >= 2) {
+                    out[1 % NO][r] += y[0][r] * acc[1 % NA][nt][r];
+                    out[2 % NO][r] += y[1 % PGH][r] * acc[0][nt][r];
+                    out[3 % NO][r] += y[0][r] * acc[2 % NA][nt][r];
+                }
+                if (PGH >= 3) {
+                    out[4 % NO][r] += y[0][r] * acc[3 % NA][nt][r];
+                    out[5 % NO][r] += y[2 % PGH][r] * acc[0][nt][r];
+                    out[6 % NO][r] += y[0][r] * acc[5 % NA][nt][r];
+                    out[7 % NO][r] += y[1 % PGH][r] * acc[1 % NA][nt][r];
+                    out[8 % NO][r] += y[0][r] * acc[4 % NA][nt][r];
+                    out[9 % NO][r] += y[1 % PGH][r] * acc[2 % NA][nt][r];
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < NO; ++k)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int o = 1; o < 16; o <<= 1) out[k][r] += __shfl_xor(out[k][r], o, 64);
+        if (wpt > 1) {
+            // the shares of the column tiles, added in order
+            if (act && sub > 0 && i16 == 0)
+#pragma unroll
+                for (int k = 0; k < NO; ++k)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) red[(w * NO + k) * 16 + k4 + 4 * r] = out[k][r];
+            __syncthreads();
+            if (act && sub == 0 && i16 == 0)
+                for (int q = 1; q < min(wpt, NB); ++q)
+#pragma unroll
+                    for (int k = 0; k < NO; ++k)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            out[k][r] += red[((w + q) * NO + k) * 16 + k4 + 4 * r];
+        }
+        if (act && sub == 0 && i16 == 0)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const long i = t0 + k4 + 4 * r;
+                if (i >= p1) continue;
+                a.pot[i * a.nd + a.ind] += 2 * out[0][r];
+                if (PGH >= 2) {
+                    const long gi = i * 3 * a.nd + a.ind;
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+                        a.grad[gi + k * a.nd] += 2 * out[(1 + k) % NO][r] * a.dsq;
+                }
+                if (PGH >= 3) {
+                    const long hi2 = i * 6 * a.nd + a.ind;
+                    const double d2 = a.dsq * a.dsq;
+#pragma unroll
+                    for (int k = 0; k < 6; ++k)
+                        a.hess[hi2 + k * a.nd] += 2 * out[(4 + k) % NO][r] * d2;
+                }
+            }
+    }
+}
+
+template <int NB, int PGH>
+static void eval3_top_launch(const Top3Args& a, hipStream_t s)
+{
+    constexpr int CS = 16 * NB + 1;
+    constexpr int NO = PGH == 1 ? 1 : (PGH == 2 ? 4 : 10);
+    const size_t lds = (4 * NO * 16 + (size_t)2 * 2 * 4 * ((a.npw + 3) / 4) * CS) * sizeof(double);
+    allow_lds3(k_eval3_top<NB, PGH>, lds);
+    // a multiple of 8 blocks: the kernel's run per die
+    klaunch(KID_EVAL_TOP, k_eval3_top<NB, PGH>, dim3((a.grid + 15) / 8 * 8), dim3(256),
+            (unsigned)lds, s, a);
+}
+
+template <int NB>
+static void eval3_top_pgh(const Top3Args& a, hipStream_t s)
+{
+    if (a.ifpgh >= 3)
+        eval3_top_launch<NB, 3>(a, s);
+    else if (a.ifpgh == 2)
+        eval3_top_launch<NB, 2>(a, s);
+    else
+        eval3_top_launch<NB, 1>(a, s);
+}
+
+void launch_eval3_top(const Top3Args& a, hipStream_t s)
+{
+    if (a.ntop <= 0) return;
+    const int nb = (a.npw + 15) / 16;
+    if (a.npw < 2 || nb > 4) fail(-3, "3D plane-wave length above 64");
+    switch (nb) {
+    case 1: eval3_top_pgh<1>(a, s); break;
+    case 2: eval3_top_pgh<2>(a, s); break;
+    case 3: eval3_top_pgh<3>(a, s); break;
+    default: eval3_top_pgh<4>(a, s); break;
+    }
+}
+
+// The leaf rank of every sorted point and the leaves' records: a wavefront
+// per leaf.
+__global__ __launch_bounds__(256) void k_top_leaves(Top3Args a, const int* __restrict__ ls,
+                                                    const int* __restrict__ ls2, int nleaves,
+                                                    const int* __restrict__ leaf_of_rank,
+                                                    const int* __restrict__ lev,
+                                                    const int* __restrict__ par,
+                                                    int* __restrict__ pb, int* __restrict__ pb2,
+                                                    TopRec* __restrict__ rec)
+{
+    const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (r >= nleaves) return;
+    const int b = leaf_of_rank[r], l = lev[b], d = l - a.ltop;
+    if (d < 0) return;  // above the cutoff level: no expansions
+    const int s0 = ls[r], s1 = ls[r + 1], t0 = ls2 ? ls2[r] : 0, t1 = ls2 ? ls2[r + 1] : 0;
+    for (int i = s0 + lane; i < s1; i += 64) pb[i] = r;
+    if (pb2)
+        for (int i = t0 + lane; i < t1; i += 64) pb2[i] = r;
+    if (lane != 0) return;
+    int top = b;
+    for (int k = 0; k < d; ++k) top = par[top];
+    TopRec q;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        q.c[k] = a.cen[3 * (long)b + k];
+        // the leaf's place among the 2^d boxes of its level along the axis
+        const int pos = (int)rint((q.c[k] - a.cen[3 * (long)top + k]) * a.ib[l] +
+                                  0.5 * ((1 << d) - 1));
+        q.row[k] = ((1 << d) - 1 + pos) * (a.npw / 2);
+    }
+    // plane-wave route: formation up to thresh sources, evaluation below
+    // thresh points
+    const int th = a.thresh[l], n = s1 - s0;
+    q.mf = th > 0 && (th == INT_MAX || n <= th) ? -1 : a.m[l];
+    q.me = th > 0 && (th == INT_MAX || n + (t1 - t0) < th) ? -1 : a.m[l];
+    rec[r] = q;
+}
+
+void launch_top_leaves(const Top3Args& a, const int* ls, const int* ls2, int nleaves,
+                       const int* leaf_of_rank, const int* lev, const int* par, int* pb, int* pb2,
+                       TopRec* rec, hipStream_t s)
+{
+    if (nleaves <= 0) return;
+    k_top_leaves<<<(nleaves + 3) / 4, 256, 0, s>>>(a, ls, ls2, nleaves, leaf_of_rank, lev, par, pb,
+                                                   pb2, rec);
 }
 
 // ---------------------------------------------------------------------------
