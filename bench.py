@@ -79,6 +79,10 @@ def per_unit(kernel, npw, nd, p, level=-1, mixed=False, keybits=18):
         return (mf if p + 1 <= 32 else "mfma"), 2.0 * (p + 1) ** 2 * nd, "flop per evaluation point"
     if kernel == "pw_eval":
         return "mfma", (8.0 * half * npw + 8.0 * npw) * nd, "flop per evaluation point"
+    if kernel in ("form_top", "eval_top"):
+        # whole cutoff-level boxes: npw real rows by npw real columns a point
+        return "mfma", 2.0 * npw * npw * nd, "flop per %s" % (
+            "source" if kernel == "form_top" else "evaluation point")
     if kernel in ("merge", "m2l", "split"):
         return "hbm", (24.0 if mixed else 48.0) * half * npw * nd, "bytes per box"
     if kernel == "gather":
@@ -134,6 +138,10 @@ def rocprof_name(kernel, nl, ifpgh, mixed=False, npw=0, sort=4):
         if nl + 1 <= 48 and npw <= 64:
             return "k_pw2local_wave<%d, %d, %s>" % (tm, (npw // 2 + 15) // 16, tt)
         return "k_pw2local<%s>" % tt
+    if kernel == "form_top":
+        return "k_form2_top<%d, false>" % ((npw + 15) // 16)
+    if kernel == "eval_top":
+        return "k_eval2_top<%d, %d>" % ((npw + 15) // 16, ifpgh)
     if kernel == "pw_eval":
         return "k_pw_eval_mfma<%d, %s>" % (ifpgh, "float" if mixed else "double")
     if kernel == "gather":

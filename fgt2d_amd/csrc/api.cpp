@@ -174,8 +174,9 @@ struct Tables2D {
     bool valid = false;
     int npw = 0, ntermmax = 0, nmax = 0;
     double pmax = 0, xmin2 = 0, xm = 0;
-    const double *ts = nullptr, *h2x = nullptr, *h2xr = nullptr, *x2l = nullptr, *rsq = nullptr,
-                 *wms = nullptr, *wm2l = nullptr;
+    const double *ws = nullptr, *ts = nullptr, *h2x = nullptr, *h2xr = nullptr, *x2l = nullptr,
+                 *rsq = nullptr, *wms = nullptr, *wm2l = nullptr;
+    const double* shift = nullptr;  // as Tables3D, for the positive nodes
     const float *wms32 = nullptr, *wm2l32 = nullptr;  // the same factors rounded to FP32
 };
 
@@ -796,6 +797,23 @@ size_t pack_leaf_keys(Pack& pk, Workspace& W, const TreeD<D>& T, int nlmax, bool
 // shift lengths), so they stay resident and are rebuilt only when those
 // change.
 // ---------------------------------------------------------------------------
+// e^{i ts_a off} of the leaves d = 0..nmax levels below a cutoff-level box of
+// scaled size xm: place q of 2^d along an axis is (q + 1/2) xm/2^d - xm/2 off
+// its centre; complex, at (2^d - 1 + q) half + a
+std::vector<double> leaf_shifts(const double* ts, int half, int nmax, double xm)
+{
+    std::vector<double> v;
+    if (nmax > TOP_DEPTH) return v;  // not on the whole-box route
+    for (int d = 0; d <= nmax; ++d)
+        for (int q = 0; q < (1 << d); ++q)
+            for (int a = 0; a < half; ++a) {
+                const double off = xm * (2 * q + 1 - (1 << d)) / (double)(2 << d);
+                v.push_back(std::cos(ts[a] * off));
+                v.push_back(std::sin(ts[a] * off));
+            }
+    return v;
+}
+
 const Tables2D& tables2d(Workspace& W, int npw, double pmax, int ntermmax, int nmax, double xmin2,
                          double xm, hipStream_t s)
 {
@@ -873,11 +891,13 @@ const Tables2D& tables2d(Workspace& W, int npw, double pmax, int ntermmax, int n
                     wm2l[o + 1] = xr * yi + xi * yr;
                 }
     std::vector<float> wms32(wms.begin(), wms.end()), wm2l32(wm2l.begin(), wm2l.end());
+    const std::vector<double> shift = leaf_shifts(ts.data(), half, nmax, xm);
     Pack pk;
     size_t o_ts = pk.add(ts), o_h2x = pk.add(h2x), o_h2xr = pk.add(h2xr), o_x2l = pk.add(x2l),
            o_rsq = pk.add(rsq);
     size_t o_wms = pk.add(wms), o_wm2l = pk.add(wm2l);
     size_t o_wms32 = pk.add(wms32), o_wm2l32 = pk.add(wm2l32);
+    size_t o_ws = pk.add(ws), o_sh = pk.add(shift);
     char* d = W.get<char>("tables", pk.size());
     HIPCHECK(hipMemcpyAsync(d, pk.data(), pk.size(), hipMemcpyHostToDevice, s));
     HIPCHECK(hipStreamSynchronize(s));  // pk is freed on return
@@ -890,6 +910,8 @@ const Tables2D& tables2d(Workspace& W, int npw, double pmax, int ntermmax, int n
     t.wm2l = (const double*)(d + o_wm2l);
     t.wms32 = (const float*)(d + o_wms32);
     t.wm2l32 = (const float*)(d + o_wm2l32);
+    t.ws = (const double*)(d + o_ws);
+    t.shift = (const double*)(d + o_sh);
     t.npw = npw; t.pmax = pmax; t.ntermmax = ntermmax; t.nmax = nmax; t.xmin2 = xmin2; t.xm = xm;
     t.valid = true;
     return t;
@@ -972,17 +994,7 @@ const Tables3D& tables3d(Workspace& W, int npw, double pmax, int ntermmax, int n
         wm1[2 * (3 * j + 1)] = 1;  wm1[2 * (3 * j + 1) + 1] = 0;    // offset 0
         wm1[2 * (3 * j + 2)] = zr; wm1[2 * (3 * j + 2) + 1] = zi;   // offset +1
     }
-    // a box d levels below the top one (size xm, scaled) at place q of 2^d
-    // along an axis is (q + 1/2) xm/2^d - xm/2 off its centre
-    std::vector<double> shift;
-    if (nmax <= TOP_DEPTH)
-        for (int d = 0; d <= nmax; ++d)
-            for (int q = 0; q < (1 << d); ++q)
-                for (int a = 0; a < half; ++a) {
-                    const double off = xm * (2 * q + 1 - (1 << d)) / (double)(2 << d);
-                    shift.push_back(std::cos(ts[a] * off));
-                    shift.push_back(std::sin(ts[a] * off));
-                }
+    const std::vector<double> shift = leaf_shifts(ts.data(), half, nmax, xm);
     Pack pk;
     size_t o_ws = pk.add(ws), o_ts = pk.add(ts), o_c = pk.add(coef), o_d = pk.add(dcoef);
     size_t o_ms = pk.add(wms), o_ml = pk.add(wm1), o_sh = pk.add(shift);
@@ -1025,6 +1037,66 @@ void zero_outputs(const Call& q, int dim, hipStream_t s)
         if (q.ifpghtarg >= 2) launch_zero(q.gradtarg, ng * nd * q.nt, s);
         if (q.ifpghtarg >= 3) launch_zero(q.hesstarg, nh * nd * q.nt, s);
     }
+}
+
+// Route of a 2D transform with expansions: whole cutoff-level boxes at once
+// (k_form2_top, k_eval2_top) or leaf by leaf, whichever the estimate below
+// finds faster; *most: the sources of the fullest refined box.  As in 3D the
+// first costs the same for a point of any leaf and the second for any leaf of
+// points, and a box's sources are one block's serial sum; but a 2D leaf is
+// cheap (wavefront kernels on both sides of the conversions), so the line lies
+// where leaves are small and boxes many.  The constants (ns) are fits to both
+// routes over uniform and mixture points, 3*10^3 to 2*10^6 of them, delta
+// 1e-5..1e-2, eps 1e-3, 1e-6, 1e-9.  Measured (by leaves -> at once): 10^5
+// uniform points, delta 1e-4, eps 1e-9 (47 a leaf): 0.46 -> 0.38 ms, 10^6 of
+// them (119 a leaf): 0.89 -> 1.00 ms, so there by leaves; 10^6 with gradients,
+// delta 6.8e-6, eps 5e-11 (orders above 32): 4.5 -> 2.1 ms; 10^5 mixture points
+// with delta 1e-4, eps 1e-6 (boxes of up to 7000): 0.40 -> 0.59 ms, by leaves.
+// FP64 only, and series of at most TOP_RF terms.
+bool top_route2(const std::vector<LeafRun>& leaves, const Call& q, int ltop, int npwlevel,
+                int nlevels, const std::vector<double>& bsz, int* most)
+{
+    if (nlevels - ltop > TOP_DEPTH || nlevels >= TOP_LEVELS) return false;
+    const int nadd = (q.rn ? 1 : 0) + std::max(q.ifpgh, q.ifpghtarg);
+    double pmax = 0;
+    int npw = 0;
+    planewave_terms(2 * bsz[0] / std::pow(2.0, ltop), q.delta, nadd > 2 ? q.eps / 100 : q.eps, &pmax,
+                    &npw);
+    if (npw < 2 || npw > 64) return false;
+    const double n2 = (double)npw * npw;
+    double cost[TOP_LEVELS], point[TOP_LEVELS];
+    int ntm = 0;
+    for (int l = ltop; l <= nlevels; ++l) {
+        int m = hermite_terms(2, bsz[l], q.delta, q.eps) + 1;
+        if (q.rn || q.ifpgh >= 2 || q.ifpghtarg >= 2) m += nadd;
+        ntm = std::max(ntm, m - 1);
+        if (l >= std::max(npwlevel + 1, 0) && m > TOP_RF) return false;
+        cost[l] = (m <= 32 ? 0.025 : 0.06) * n2;
+        point[l] = m <= 32 ? 0.1 * (m / 20.0) * (m / 20.0) : 1.0;
+    }
+    if (g_precision == 1 && q.eps >= kMixedEpsMin && ntm < 63) return false;
+    double leafwise = 7e4, nsum = 0;
+    int here = 0;
+    uint64_t last = ~(uint64_t)0;
+    *most = 0;
+    const size_t n = leaves.size();
+    for (size_t i = 0; i < n; ++i) {
+        const int l = leaves[i].level;
+        if (l < ltop || l <= npwlevel) continue;
+        const int c = (i + 1 < n ? leaves[i + 1].start : q.ns) - leaves[i].start;
+        const uint64_t box = leaves[i].key >> (2 * (l - ltop));
+        here = box == last ? here + c : c;
+        last = box;
+        *most = std::max(*most, here);
+        leafwise += cost[l] + point[l] * c;
+        nsum += c;
+    }
+    auto weight = [](int ifpgh) { return ifpgh <= 0 ? 0.0 : (ifpgh == 1 ? 1.0 : (ifpgh == 2 ? 3.0 : 6.0)); };
+    // evaluated points as if spread like the sources
+    const double et = q.ifpghtarg > 0 ? (double)q.nt / q.ns : 0.0;
+    const double form = std::max((0.1 + 8e-5 * n2) * nsum, (15 + 0.06 * n2) * *most) * (q.rn ? 2.5 : 1.0);
+    const double eval = (0.1 + 1.3e-4 * n2) * nsum * (weight(q.ifpgh) + et * weight(q.ifpghtarg));
+    return form + eval < leafwise;  // every density costs the same again
 }
 
 void run2d(Workspace& W, const Call& q, hipStream_t s)
@@ -1239,8 +1311,10 @@ void run2d(Workspace& W, const Call& q, hipStream_t s)
     std::vector<double> bsz0(L0 + 1);
     bsz0[0] = bs0;
     for (int l = 0; l < L0; ++l) bsz0[l + 1] = bsz0[l] / 2;  // as the builder halves
+    int most = 0;
+    const bool top0 = npwlevel < L0 && top_route2(leaves, q, nlevstart, npwlevel, L0, bsz0, &most);
     const bool early_ok = !g_serial && !tm.on && !W.arena && npwlevel < L0 && L0 >= 1 &&
-                          L0 >= std::max(npwlevel + 1, 0);
+                          L0 >= std::max(npwlevel + 1, 0) && !top0;
     struct Early {
         bool on = false;
         int nL = 0, nl = 0, npw = 0;
@@ -1385,14 +1459,19 @@ void run2d(Workspace& W, const Call& q, hipStream_t s)
     const bool mixed = g_precision == 1 && expansions && q.eps >= kMixedEpsMin && ntermmax < 63;
     const size_t esz = mixed ? sizeof(float) : sizeof(double);
 
+    // the cutoff-level boxes formed and evaluated whole (k_form2_top, k_eval2_top)
+    const bool top = top0 && expansions && nlevels == L0;
+
     // box arrays; expansion slots: the finest level first (its leaves are
     // formed first, possibly before the tree), then the other levels from
-    // the cutoff level down
+    // the cutoff level down; the cutoff level alone on the whole-box route
     std::vector<int>& slot = W.h_slot;
     slot.assign(nb, -1);
     int nslot = 0;
     const int bL0 = T.laddr[2 * nlevels], bL1 = T.laddr[2 * nlevels + 1], nL = bL1 - bL0 + 1;
-    if (expansions) {
+    if (top) {
+        for (int b = T.laddr[2 * nlevstart]; b <= T.laddr[2 * nlevstart + 1]; ++b) slot[b] = nslot++;
+    } else if (expansions) {
         for (int b = bL0; b <= bL1; ++b) slot[b] = nslot++;
         for (int b = 0; b < bL0; ++b)
             if (T.lev[b] >= nlevstart) slot[b] = nslot++;
@@ -1445,7 +1524,7 @@ void run2d(Workspace& W, const Call& q, hipStream_t s)
             }
         const int* nch = T.nch.data();
         const int* ch = T.ch.data();
-        for (int l = 0; l <= nlevels; ++l) {
+        for (int l = 0; l <= (top ? nlevstart : nlevels); ++l) {
             const int b0 = T.laddr[2 * l], b1 = T.laddr[2 * l + 1];
             const bool fl = l >= std::max(npwlevel + 1, 0), el = l >= nlevstart,
                        ml = l >= nlevstart && l <= nlevels - 1;
@@ -1454,7 +1533,11 @@ void run2d(Workspace& W, const Call& q, hipStream_t s)
             std::vector<int>& sp = split_l[l];
             std::vector<int>& e = eval_l[l];
             for (int b = b0; b <= b1; ++b) {
-                if (nch[b] == 0) {
+                if (top && l == nlevstart && nch[b] > 0) {
+                    // formed and evaluated with every leaf below
+                    f.push_back(b);
+                    e.push_back(b);
+                } else if (nch[b] == 0) {
                     if (fl) f.push_back(b);
                     if (el && !(l == npwlevel && !iflocal[b]))
                         e.push_back(b);
@@ -1476,6 +1559,8 @@ void run2d(Workspace& W, const Call& q, hipStream_t s)
         }
         o_m2l = pk.add(m2l_l);
     }
+    size_t o_lev = 0, o_lofr = 0;
+    if (top) o_lev = pk.add(T.lev), o_lofr = pk.add(T.leaf_of_rank);
     const size_t o_resid = pk.add(resid);
     const Tables2D& tab = expansions ? tables2d(W, npw, pmax, ntermmax, nlevels - nlevstart,
                                                 T.bsz[nlevels] / std::sqrt(q.delta) / 2,
@@ -1578,7 +1663,7 @@ void run2d(Workspace& W, const Call& q, hipStream_t s)
     const size_t nexp_d = per * nslot * esz / sizeof(double);  // per is even
     // the finest level's leaves store their expansions (no clearing); the
     // other boxes accumulate (merges)
-    const size_t nfin_d = expansions ? per * nL * esz / sizeof(double) : 0;
+    const size_t nfin_d = expansions && !top ? per * nL * esz / sizeof(double) : 0;
     if (expansions) launch_zero3(nullptr, 0, mp + nfin_d, nexp_d - nfin_d, lc, nexp_d, s_g);
     auto D = [&](size_t off) { return (void*)(dplan + off); };
     const int4* d_child = (const int4*)D(o_child);
@@ -1706,7 +1791,103 @@ void run2d(Workspace& W, const Call& q, hipStream_t s)
     };
 
     // ---------------- expansions: steps 1-5 ----------------
-    if (expansions) {
+    if (top) {
+        const std::vector<int>&form = form_l[nlevstart], &ev = eval_l[nlevstart];
+        const size_t nte = ev.size(), sg_t = nte + nt / TOP2_SEG + 1, sg_s = nte + ns / TOP2_SEG + 1;
+        int* seg_t = W.get<int>("tstart", 2 * (nte + 1));
+        int* seg_s = seg_t + nte + 1;
+        int* box_t = W.get<int>("segbox", sg_t + sg_s);
+        int* box_s = box_t + sg_t;
+        const int* d_ev = (const int*)D(o_eval[nlevstart]);
+        SegLists L{};
+        if (use_trg) L.l[L.count++] = SegList{d_ev, (int)nte, trg_se, TOP2_SEG, seg_t, box_t};
+        if (use_src) L.l[L.count++] = SegList{d_ev, (int)nte, src_se, TOP2_SEG, seg_s, box_s};
+        launch_seg_scan(L, s);
+        TopLeafArgs la{};
+        la.ls = ls;
+        la.ls2 = tg ? ls2 : nullptr;
+        la.nleaves = nleaves;
+        la.leaf_of_rank = (const int*)D(o_lofr);
+        la.lev = (const int*)D(o_lev);
+        la.par = d_par;
+        la.cen = d_cen;
+        la.ltop = nlevstart;
+        la.half = half;
+        for (int l = nlevstart; l <= nlevels; ++l) {
+            la.m[l] = nlocal[l] + 1;
+            la.eth[l] = nlocal[l] > 50 ? INT_MAX : 0;  // nlocalswitch, fgt2d.f:855
+            la.ib[l] = 1.0 / T.bsz[l];
+        }
+        // leaf of every sorted point, in place of arrays that are free by now
+        la.pb = lvl;
+        la.pb2 = use_trg ? (int*)W.get<u64>("keys_t", nt) : nullptr;
+        la.rec = W.get<TopRec>("leaf_rec", nleaves);
+        launch_top_leaves2(la, s);
+        Top2Args ta{};
+        ta.rec = la.rec;
+        ta.nd = nd;
+        ta.dsq = dsq;
+        ta.npw = npw;
+        ta.ws = tab.ws;
+        ta.ts = tab.ts;
+        ta.shift = (const double2*)tab.shift;
+        ta.nshift = ((2 << (nlevels - nlevstart)) - 1) * half;
+        ta.slot = d_slot;
+        tm.begin(S_FORM);
+        Top2Args fa = ta;
+        fa.tops = (const int*)D(o_form[nlevstart]);
+        fa.ntop = (int)form.size();
+        fa.se = src_se;
+        fa.pbox = la.pb;
+        fa.pts = xs;
+        fa.qs = qs;
+        fa.dipw = wsd;
+        fa.exp = mp;
+        fa.waves = most > 512 ? 8 : 4;  // few sources: more boxes per CU instead (100k: 43 -> 39 us)
+        tm.ctx(nlevstart, &form, 0);
+        launch_form2_top(fa, s);
+        tm.end(S_FORM);
+        near_field_if_ready();
+        tm.begin(S_M2L);
+        tm.ctx(nlevstart, &m2l_l, 2);
+        launch_m2l((const int*)D(o_m2l), (int)m2l_l.size(), d_cen, d_ncol, d_col, src_se, trg_se,
+                   use_src, use_trg, d_slot, tab.wm2l, npwlevel >= 0 ? T.bsz[npwlevel] : T.bsz[0],
+                   nlevstart == npwlevel, nd, nexp, mp, lc, s, false);
+        tm.end(S_M2L);
+        // every evaluation adds the near field's outputs
+        if (!nf_queued) near_field();
+        tm.begin(S_EVAL);
+        W.wait(s, nf_ready);
+        for (int side = 0; side < 2; ++side) {
+            if (side == 0 ? !use_trg : !use_src) continue;
+            Top2Args ea = ta;
+            ea.tops = d_ev;
+            ea.ntop = (int)nte;
+            ea.se = side == 0 ? trg_se : src_se;
+            ea.pbox = side == 0 ? la.pb2 : la.pb;
+            ea.pts = side == 0 ? xt : xs;
+            ea.exp = lc;
+            ea.tstart = side == 0 ? seg_t : seg_s;
+            ea.segbox = side == 0 ? box_t : box_s;
+            ea.grid = (int)std::min<size_t>(1 << 16, side == 0 ? sg_t : sg_s);
+            EvalArgs eb{};
+            eb.nd = nd;
+            eb.ifpgh = side == 0 ? q.ifpghtarg : q.ifpgh;
+            eb.pot = side == 0 ? q.pottarg : q.pot;
+            eb.grad = side == 0 ? q.gradtarg : q.grad;
+            eb.hess = side == 0 ? q.hesstarg : q.hess;
+            eb.perm = side == 0 ? itarg : isrc;
+            eb.npot = side == 0 ? npt : nps;
+            eb.ngrad = side == 0 ? ngt : ngs;
+            eb.nhess = side == 0 ? nht : nhs;
+            for (int ind = 0; ind < nd; ++ind) {
+                eb.ind = ind;
+                tm.ctx(nlevstart, &ev, side == 0 ? 1 : 0);
+                launch_eval2_top(ea, eb, s);
+            }
+        }
+        tm.end(S_EVAL);
+    } else if (expansions) {
         const double* d_h2x = tab.h2x;
         const double* d_h2xr = tab.h2xr;
         const double* d_x2l = tab.x2l;
@@ -2725,18 +2906,29 @@ void run3d(Workspace& W, const Call& q, hipStream_t s)
         ta.nd = nd;
         ta.dsq = dsq;
         ta.npw = npw;
-        ta.ltop = nlevstart;
         ta.ws = tab.ws;
         ta.ts = tab.ts;
         ta.shift = (const double2*)tab.shift;
         ta.nshift = ((2 << (nlevels - nlevstart)) - 1) * half;
+        TopLeafArgs la{};
+        la.ls = ls;
+        la.ls2 = tg ? ls2 : nullptr;
+        la.nleaves = nleaves;
+        la.leaf_of_rank = (const int*)D(o_lofr);
+        la.lev = (const int*)D(o_lev);
+        la.par = d_par;
+        la.cen = d_cen;
+        la.ltop = nlevstart;
+        la.half = half;
         for (int l = nlevstart; l <= nlevels; ++l) {
-            ta.m[l] = nlocal[l] + 1;
-            ta.thresh[l] = form_thresh[l];
-            ta.ib[l] = 1.0 / T.bsz[l];
+            la.m[l] = nlocal[l] + 1;
+            la.fth[l] = la.eth[l] = form_thresh[l];
+            la.ib[l] = 1.0 / T.bsz[l];
         }
-        launch_top_leaves(ta, ls, tg ? ls2 : nullptr, nleaves, (const int*)D(o_lofr),
-                          (const int*)D(o_lev), d_par, pb_s, pb_t, rec, s);
+        la.pb = pb_s;
+        la.pb2 = pb_t;
+        la.rec = rec;
+        launch_top_leaves(la, s);
         tm.begin(S_FORM);
         for (int ind = 0; ind < nd; ++ind) {
             Top3Args fa = ta;

@@ -284,6 +284,60 @@ void launch_pw2local(const EvalArgs& a, hipStream_t s);
 void launch_taylor_eval(const EvalArgs& a, hipStream_t s);
 void launch_pw_eval(const EvalArgs& a, hipStream_t s);
 
+// ---------------------------------------------------------------------------
+// Formation and evaluation of whole cutoff-level boxes (2D and 3D): the
+// leaves' truncated series about their centres, moved to the box's centre
+// ---------------------------------------------------------------------------
+constexpr int TOP_LEVELS = 32, TOP_DEPTH = 4;  // levels; of these below the cutoff level
+constexpr int TOP_RF = 66;                     // most terms of a truncated series
+struct TopRec {             // one leaf, as the phase tables need it
+    double c[3];            // centre
+    int row[3];             // shift table rows per axis (offset of node 0)
+    int mf, me;             // terms of its series, formation and evaluation; -1: whole exponentials
+};
+// Per sorted point (sources ls, targets ls2 or nullptr) its leaf's rank, into
+// pb and pb2, and per leaf rank its record.
+struct TopLeafArgs {
+    const int *ls, *ls2;
+    int nleaves;
+    const int *leaf_of_rank, *lev, *par;
+    const double* cen;
+    int ltop, half;         // the cutoff level; nodes per shift table row
+    // per level: terms of the series, thresholds of the plane-wave route
+    // (formation up to fth sources, evaluation below eth points; 0 never,
+    // INT_MAX always), 1 / box size
+    int m[TOP_LEVELS], fth[TOP_LEVELS], eth[TOP_LEVELS];
+    double ib[TOP_LEVELS];
+    int *pb, *pb2;
+    TopRec* rec;
+};
+struct Top2Args {
+    const int* tops;        // cutoff-level boxes
+    int ntop;
+    const int2* se;         // point ranges of the boxes (sources, or the evaluated points)
+    const int* pbox;        // leaf rank of every sorted point
+    const TopRec* rec;
+    const double* pts;      // sorted points
+    const double* qs;       // formation: sorted charges (n, nd)
+    const double* dipw;     // formation: dipole weights d n, (n, nd, 2) sorted, or nullptr
+    int nd;
+    double dsq;
+    int npw;
+    const double *ws, *ts;  // nodes: npw/2 positive ones, then their mirrors
+    const double2* shift;   // e^{i ts_a (c_leaf - c_top)}, a < npw/2: rows 2^d - 1 + place
+    int nshift;             // along the axis, d levels below the top; entries of the table
+    const int* slot;
+    double* exp;            // complex per slot (nd, nexp): written, or read by the evaluation
+    // evaluation: segments of TOP2_SEG points (as SegList), outputs as EvalArgs
+    const int *tstart, *segbox;
+    int grid;
+    int waves;              // formation: wavefronts per box, 1 to 8
+};
+constexpr int TOP2_SEG = 256;
+void launch_top_leaves2(const TopLeafArgs& a, hipStream_t s);
+void launch_form2_top(const Top2Args& a, hipStream_t s);
+void launch_eval2_top(const Top2Args& a, const EvalArgs& e, hipStream_t s);
+
 struct DirectArgs {
     const int* units;       // target units (boxes)
     int nunits;
@@ -356,12 +410,6 @@ long form3_mfma_scratch(int m, int npw);  // per-block scratch of the matrix-cor
 void launch_form3_pw(const Form3Args& a, hipStream_t s);
 
 // Formation and evaluation at the cutoff level (k_form3_top, k_eval3_top)
-constexpr int TOP_LEVELS = 24, TOP_DEPTH = 4;  // levels; of these below the cutoff level
-struct TopRec {             // one leaf, as the phase tables need it
-    double c[3];            // centre
-    int row[3];             // shift table rows per axis (offset of node 0)
-    int mf, me;             // terms of its series, formation and evaluation; -1: whole exponentials
-};
 struct Top3Args {
     const int* tops;        // cutoff-level boxes
     int ntop;
@@ -374,16 +422,12 @@ struct Top3Args {
     const double* dipw;     // formation: dipole weights d n, (n, nd, 3) sorted, or nullptr
     int nd, ind;
     double dsq;
-    int npw, ltop;
+    int npw;
     const double *ws, *ts;  // nodes (ascending)
     const double2* shift;   // e^{i ts_a (c_leaf - c_top)}, a < npw/2: rows 2^d - 1 + place
     int nshift;             // along the axis, d levels below the top; entries of the table
     const int* slot;
     double* mp;             // per slot (nd, nexp) complex: written, or read by the evaluation
-    // per level: terms of the leaves' series, route threshold (as Form3Args,
-    // Eval3Args), 1 / box size
-    int m[TOP_LEVELS], thresh[TOP_LEVELS];
-    double ib[TOP_LEVELS];
     // evaluation: segments of 64 points (tstart, segbox as SegList), outputs
     // accumulated
     const int *tstart, *segbox;
@@ -392,11 +436,7 @@ struct Top3Args {
 };
 void launch_form3_top(const Top3Args& a, hipStream_t s);
 void launch_eval3_top(const Top3Args& a, hipStream_t s);
-// pb[i] = r for the sources ls[r] <= i < ls[r + 1] of every leaf rank (pb2:
-// the targets of ls2, or nullptr), and the leaves' records
-void launch_top_leaves(const Top3Args& a, const int* ls, const int* ls2, int nleaves,
-                       const int* leaf_of_rank, const int* lev, const int* par, int* pb, int* pb2,
-                       TopRec* rec, hipStream_t s);
+void launch_top_leaves(const TopLeafArgs& a, hipStream_t s);
 
 void launch_merge3(const int* parents, int np, const int* child8, const double* cen,
                    const int2* src_se, const int* slot, const double* wms, int kbase, int nd,

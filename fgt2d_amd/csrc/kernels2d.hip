@@ -19,6 +19,7 @@
 #include <rocprim/iterator/counting_iterator.hpp>
 
 #include "fgtpw_impl.hpp"
+#include "top_phase.hpp"
 
 namespace fgtpw {
 
@@ -3218,6 +3219,405 @@ __device__ __forceinline__ void pair_add(double dx, double dy, double q, double 
             hyy += e * ((rfac + uy * uy) * A - (DIP ? 2.0 * rfac * uy * w2 : 0.0));
         }
     }
+}
+
+// ---------------------------------------------------------------------------
+// Formation (steps 1-2) and evaluation (steps 4-5) of whole cutoff-level
+// boxes in FP64.  Each axis' truncated exponential about a leaf's centre,
+// moved to the cutoff-level box's centre, is the real pair (C, S)(x, a),
+// a < npw/2 (top_phase.hpp); mirror nodes are conjugates, so
+//   mp(a, +-b) = sum_s q (C - iS)(x,a) (C -+ iS)(y,b) ws_a ws_b
+//   pot(p)     = 2 Re sum (C + iS)(x,a) (C +- iS)(y,b) loc(a, +-b)
+// are one real npw x npw product each over the box's points: 2 npw^2
+// operations a point, on FP64 matrix cores, and no leaf expansion is formed,
+// merged, split or converted.  A lane builds its operands itself: it computes
+// the pair of one node and supplies the cosine to one 16-wide tile and the
+// sine to the next (nodes in groups of 16; a last group of at most 8 shares
+// one tile, cosines in lanes 0-7, sines in 8-15).  Bound by the series (FP64
+// VALU) and latency; the matrix pipe is 20-25% busy.  Against the leaf kernels
+// they replace, us: 10^6 uniform points with gradients, eps 5e-11 (npw 44,
+// leaves of order 37 and 24): formation and merge 1600 -> 335, conversion,
+// split and evaluation 2250 -> 800; 10^5, eps 1e-9 (npw 38): 120 -> 42 and
+// 86 -> 46.
+// ---------------------------------------------------------------------------
+// place of (node, sine or cosine) among the 16 NB rows or columns
+template <int NB>
+__device__ __forceinline__ int top2_place(int node, int sn)
+{
+    constexpr int F = 16 * (NB / 2);  // nodes in full groups
+    if (!(NB & 1) || node < F) return 32 * (node >> 4) + 16 * sn + (node & 15);
+    return 2 * F + (node - F) + 8 * sn;
+}
+// node of lane i16 in group g
+template <int NB>
+__device__ __forceinline__ int top2_node(int g, int i16)
+{
+    return (NB & 1) && g == NB / 2 ? 16 * g + (i16 & 7) : 16 * g + i16;
+}
+
+// Formation: one block of 2 to 8 wavefronts per (box, density), which take
+// groups of 4 sources in turn through the MFMA K dimension, and the
+// wavefronts' sums are added in order.  With dipoles the product gains
+// X (w2 Y') + X' (w1 Y), primes the derivatives along the axis.
+template <int NB, bool DIP>
+__global__ __launch_bounds__(512, NB <= 2 ? 4 : 2) void k_form2_top(Top2Args a)
+{
+    constexpr int NG = (NB + 1) / 2, W = 16 * NB;
+    extern __shared__ double sm[];
+    double* R = sm;                             // [16 NB][16 NB]
+    double2* shl = (double2*)(R + W * W);       // the shift table
+    const int t = threadIdx.x, w = t >> 6, lane = t & 63, i16 = lane & 15, k4 = lane >> 4;
+    const int nthr = blockDim.x, nw = nthr >> 6, step = 4 * nw;  // sources of a round
+    const int npw = a.npw, half = npw / 2, ind = blockIdx.y;
+    const int box = a.tops[blockIdx.x];
+    const int2 r = a.se[box];
+    for (int o = t; o < a.nshift; o += nthr) shl[o] = a.shift[o];
+    // this lane's nodes
+    int node[NG];
+    double tsn[NG], wsn[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        const int n = top2_node<NB>(g, i16);
+        node[g] = min(n, half - 1);
+        tsn[g] = a.ts[node[g]];
+        wsn[g] = n < half ? a.ws[node[g]] : 0.0;  // no such node: zero rows, columns
+    }
+    d4_top acc[NB][NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = (d4_top){0, 0, 0, 0};
+    __syncthreads();
+    // the next sources' places and leaves are loaded beside this one's
+    // products; past the end: the last source's place, no charge or strength
+    const int last = r.y - 1;
+    int pb = 0;
+    double px = 0, py = 0, pq = 0, pw1 = 0, pw2 = 0;
+    TopRec pr;
+    auto fetch = [&](int i0) {
+        const int i = min(i0, last);
+        const bool in = i0 <= last;
+        pr = a.rec[pb];
+        px = a.pts[2 * (long)i];
+        py = a.pts[2 * (long)i + 1];
+        const long o = (long)a.nd * i + ind;
+        pq = in ? a.qs[o] : 0.0;
+        if (DIP) {
+            pw1 = in ? a.dsq * a.dipw[2 * o] : 0.0;
+            pw2 = in ? a.dsq * a.dipw[2 * o + 1] : 0.0;
+        }
+        pb = a.pbox[min(i0 + step, last)];
+    };
+    int i0 = r.x + 4 * w + k4;
+    if (r.x < r.y) {
+        pb = a.pbox[min(i0, last)];
+        fetch(i0);
+    }
+    for (int s0 = r.x + 4 * w; s0 < r.y; s0 += step) {
+        const double ux = (px - pr.c[0]) * a.dsq, uy = (py - pr.c[1]) * a.dsq;
+        const double q = pq, w1 = pw1, w2 = pw2;
+        const int rx = pr.row[0], ry = pr.row[1], mf = pr.mf;
+        i0 += step;
+        if (s0 + step < r.y) fetch(i0);
+        double u[2 * NG];
+        int m[2 * NG];
+        double2 e[DIP ? 2 : 1][2 * NG];
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            u[g] = tsn[g] * ux;
+            u[NG + g] = tsn[g] * uy;
+            m[g] = m[NG + g] = mf;
+        }
+        top_series<2 * NG, DIP ? 2 : 1>(u, m, e);
+        double X[NB], Y[NB], X1[NB], Y1[NB];
+#pragma unroll
+        for (int g = 0; g < 2 * NG; ++g) {
+            const int gg = g % NG;
+            const double2 sh = shl[(g < NG ? rx : ry) + node[gg]];
+            const double f = wsn[gg];
+            double2 v = top_shift(e[0][g], sh), d = make_double2(0, 0);
+            v.x *= f;
+            v.y *= f;
+            if (DIP) {
+                // (C', S') = ts (-S, C) of one term fewer
+                const double2 h = top_shift(e[DIP ? 1 : 0][g], sh);
+                d = make_double2(-tsn[gg] * f * h.y, tsn[gg] * f * h.x);
+            }
+            double* o = g < NG ? X : Y;
+            double* o1 = g < NG ? X1 : Y1;
+            if ((NB & 1) && gg == NB / 2) {
+                o[2 * gg] = i16 < 8 ? v.x : v.y;
+                if (DIP) o1[2 * gg] = i16 < 8 ? d.x : d.y;
+            } else {
+                o[2 * gg] = v.x;
+                o[2 * gg + 1] = v.y;
+                if (DIP) o1[2 * gg] = d.x, o1[2 * gg + 1] = d.y;
+            }
+        }
+#pragma unroll
+        for (int nt = 0; nt < NB; ++nt) {
+            const double b = DIP ? q * Y[nt] + w2 * Y1[nt] : q * Y[nt];
+#pragma unroll
+            for (int mt = 0; mt < NB; ++mt)
+                acc[mt][nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(X[mt], b, acc[mt][nt], 0, 0, 0);
+            if (DIP) {
+                const double c = w1 * Y[nt];
+#pragma unroll
+                for (int mt = 0; mt < NB; ++mt)
+                    acc[mt][nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(X1[mt], c, acc[mt][nt], 0, 0, 0);
+            }
+        }
+    }
+    for (int q = 0; q < nw; ++q) {
+        if (w == q)
+#pragma unroll
+            for (int mt = 0; mt < NB; ++mt)
+#pragma unroll
+                for (int nt = 0; nt < NB; ++nt)
+#pragma unroll
+                    for (int rr = 0; rr < 4; ++rr) {
+                        double* p = R + (16 * mt + k4 + 4 * rr) * W + 16 * nt + i16;
+                        *p = q == 0 ? acc[mt][nt][rr] : *p + acc[mt][nt][rr];
+                    }
+        __syncthreads();
+    }
+    double2* out = (double2*)a.exp + ((long)a.slot[box] * a.nd + ind) * (long)half * npw;
+    for (int o = t; o < half * half; o += nthr) {
+        const int aa = o % half, b = o / half;
+        const double* rc = R + top2_place<NB>(aa, 0) * W;
+        const double* rs = R + top2_place<NB>(aa, 1) * W;
+        const int pc = top2_place<NB>(b, 0), ps = top2_place<NB>(b, 1);
+        const double cc = rc[pc], cs = rc[ps], sc = rs[pc], ss = rs[ps];
+        out[aa + half * b] = make_double2(cc - ss, -(sc + cs));
+        out[aa + half * (b + half)] = make_double2(cc + ss, cs - sc);
+    }
+}
+
+template <int NB, bool DIP>
+static void form2_top_launch(const Top2Args& a, hipStream_t s)
+{
+    const size_t lds = (size_t)256 * NB * NB * sizeof(double) + a.nshift * sizeof(double2);
+    klaunch(KID_FORM_TOP, k_form2_top<NB, DIP>, dim3((unsigned)a.ntop, (unsigned)a.nd),
+            dim3(64 * a.waves), (unsigned)lds, s, a);
+}
+
+void launch_form2_top(const Top2Args& a, hipStream_t s)
+{
+    if (a.ntop <= 0) return;
+    const int nb = (a.npw + 15) / 16;
+    if (a.npw < 2 || nb > 4) fail(-3, "2D plane-wave length above 64 on the whole-box route");
+    const bool dip = a.dipw != nullptr;
+    switch (nb) {
+    case 1: dip ? form2_top_launch<1, true>(a, s) : form2_top_launch<1, false>(a, s); break;
+    case 2: dip ? form2_top_launch<2, true>(a, s) : form2_top_launch<2, false>(a, s); break;
+    case 3: dip ? form2_top_launch<3, true>(a, s) : form2_top_launch<3, false>(a, s); break;
+    default: dip ? form2_top_launch<4, true>(a, s) : form2_top_launch<4, false>(a, s); break;
+    }
+}
+
+// Evaluation: one block of 4 wavefronts per segment of TOP2_SEG points of one
+// box, a wavefront per 16 points at a time.  The box's expansion is staged as
+// the real matrix R(k, col), pot = 2 X^T R Y, from the sums and differences
+// over the mirror nodes in y; T = X R on matrix cores, the y weights (and
+// derivatives) on its columns, x derivatives in rows of their own.  Values go
+// to the caller's arrays in input order with the near field added (eval_out).
+template <int NB, int PGH>
+__global__ __launch_bounds__(256, PGH > 1 ? 2 : (NB <= 2 ? 4 : (NB == 3 ? 3 : 2))) void k_eval2_top(Top2Args a, EvalArgs e)
+{
+    constexpr int NG = (NB + 1) / 2, CS = 16 * (NB | 1), NQ = 2 * NB, KS = 2 * NQ, NX = PGH;
+    constexpr int NO = PGH == 1 ? 1 : (PGH == 2 ? 3 : 6);
+    extern __shared__ double sm[];
+    double* R = sm;                              // [8 nq][CS]
+    const int t = threadIdx.x, w = t >> 6, lane = t & 63, i16 = lane & 15, k4 = lane >> 4;
+    const int npw = a.npw, half = npw / 2, nq = (half + 3) / 4;
+    double2* shl = (double2*)(R + 8 * nq * CS);  // the shift table
+    for (int o = t; o < a.nshift; o += 256) shl[o] = a.shift[o];
+    for (int o = t; o < 8 * nq * CS; o += 256) R[o] = 0.0;  // padding stays zero
+    const int total = a.tstart[a.ntop];
+    for (int g = blockIdx.x; g < total; g += gridDim.x) {
+        const int li = a.segbox[g], box = a.tops[li];
+        const int2 rr = a.se[box];
+        const int p0 = rr.x + (g - a.tstart[li]) * TOP2_SEG, p1 = min(rr.y, p0 + TOP2_SEG);
+        const double2* pw = (const double2*)a.exp + ((long)a.slot[box] * a.nd + e.ind) * (long)half * npw;
+        __syncthreads();  // the zeros; readers of the last segment's R are done
+        for (int o = t; o < half * half; o += 256) {
+            const int aa = o % half, b = o / half;
+            const double2 v = pw[aa + half * b], m = pw[aa + half * (b + half)];
+            double* rc = R + (8 * (aa >> 2) + (aa & 3)) * CS;
+            double* rs = rc + 4 * CS;
+            const int pc = top2_place<NB>(b, 0), ps = top2_place<NB>(b, 1);
+            rc[pc] = v.x + m.x;
+            rc[ps] = -(v.y - m.y);
+            rs[pc] = -(v.y + m.y);
+            rs[ps] = -(v.x - m.x);
+        }
+        __syncthreads();
+        for (int t0 = p0 + 16 * w; t0 < p1; t0 += 64) {
+            // the point whose x rows this lane supplies, and for lanes
+            // i16 < 4 the point whose values it stores
+            const long pa = min(t0 + i16, p1 - 1);
+            const TopRec L = a.rec[a.pbox[pa]];
+            const int ps = t0 + k4 + 4 * (i16 & 3);
+            const bool st = i16 < 4 && ps < p1;
+            long po = 0;
+            double nf = 0;
+            if (st) {
+                po = e.perm[ps];
+                nf = e.npot[(long)ps * e.nd + e.ind];
+            }
+            const double ux = (a.pts[2 * pa] - L.c[0]) * a.dsq, uy = (a.pts[2 * pa + 1] - L.c[1]) * a.dsq;
+            double X[NX][KS];
+            {
+                double u[NQ], tsq[NQ];
+                int m[NQ];
+                double2 f[NX][NQ];
+#pragma unroll
+                for (int j = 0; j < NQ; ++j) {
+                    m[j] = L.me;
+                    tsq[j] = a.ts[min(4 * j + k4, half - 1)];
+                    u[j] = tsq[j] * ux;
+                }
+                top_series<NQ, NX>(u, m, f);
+#pragma unroll
+                for (int d = 0; d < NX; ++d) {
+#pragma unroll
+                    for (int j = 0; j < NQ; ++j) {
+                        const int node = 4 * j + k4;
+                        const double2 v = top_shift(f[d][j], shl[L.row[0] + min(node, half - 1)]);
+                        const double z = node < half ? 1.0 : 0.0, ts = z * tsq[j];
+                        X[d][2 * j] = d == 0 ? z * v.x : (d == 1 ? -ts * v.y : -ts * tsq[j] * v.x);
+                        X[d][2 * j + 1] = d == 0 ? z * v.y : (d == 1 ? ts * v.x : -ts * tsq[j] * v.y);
+                    }
+                }
+            }
+            // pot; gx gy; hxx hxy hyy
+            double out[NO][4];
+#pragma unroll
+            for (int k = 0; k < NO; ++k)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) out[k][r] = 0;
+            double uyr[4];
+            int row[4], m0[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                uyr[r] = __shfl(uy, k4 + 4 * r, 64);
+                row[r] = __shfl(L.row[1], k4 + 4 * r, 64);
+                m0[r] = __shfl(L.me, k4 + 4 * r, 64);
+            }
+#pragma unroll
+            for (int gr = 0; gr < NG; ++gr) {
+                const int n = top2_node<NB>(gr, i16), node = min(n, half - 1);
+                const double tsn = a.ts[node];
+                const bool tail = (NB & 1) && gr == NB / 2;
+                // weights of the cosine and sine tiles, of the one shared
+                // tile in a last group
+                double yc[PGH][4], ys[PGH][4];
+                {
+                    double u[4];
+                    double2 f[PGH][4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) u[r] = tsn * uyr[r];
+                    top_series<4, PGH>(u, m0, f);
+#pragma unroll
+                    for (int d = 0; d < PGH; ++d) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const double2 v = top_shift(f[d][r], shl[row[r] + node]);
+                            const double c = d == 0 ? v.x : (d == 1 ? -tsn * v.y : -tsn * tsn * v.x);
+                            const double sv = d == 0 ? v.y : (d == 1 ? tsn * v.x : -tsn * tsn * v.y);
+                            yc[d][r] = tail && i16 >= 8 ? sv : c;
+                            ys[d][r] = sv;
+                        }
+                    }
+                }
+#pragma unroll
+                for (int sn = 0; sn < (tail ? 1 : 2); ++sn) {
+                    const int nt = 2 * gr + sn;
+                    d4_top T[NX];
+#pragma unroll
+                    for (int ix = 0; ix < NX; ++ix) T[ix] = (d4_top){0, 0, 0, 0};
+#pragma unroll
+                    for (int ks = 0; ks < KS; ++ks) {
+                        if (ks >= 2 * nq) break;
+                        const double b = R[(4 * ks + k4) * CS + 16 * nt + i16];
+#pragma unroll
+                        for (int ix = 0; ix < NX; ++ix)
+                            T[ix] = __builtin_amdgcn_mfma_f64_16x16x4f64(X[ix][ks], b, T[ix], 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        double yv[PGH];
+#pragma unroll
+                        for (int d = 0; d < PGH; ++d) yv[d] = sn ? ys[d][r] : yc[d][r];
+                        out[0][r] += yv[0] * T[0][r];
+                        if (PGH >= 2) {
+                            out[1 % NO][r] += yv[0] * T[1 % NX][r];
+                            out[2 % NO][r] += yv[1 % PGH] * T[0][r];
+                        }
+                        if (PGH >= 3) {
+                            out[3 % NO][r] += yv[0] * T[2 % NX][r];
+                            out[4 % NO][r] += yv[1 % PGH] * T[1 % NX][r];
+                            out[5 % NO][r] += yv[2 % PGH] * T[0][r];
+                        }
+                    }
+                }
+            }
+            double val[NO];
+#pragma unroll
+            for (int k = 0; k < NO; ++k) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int o = 1; o < 16; o <<= 1) out[k][r] += __shfl_xor(out[k][r], o, 64);
+                val[k] = 2 * out[k][0];
+#pragma unroll
+                for (int r = 1; r < 4; ++r)
+                    if (i16 == r) val[k] = 2 * out[k][r];
+            }
+            const double d1 = a.dsq, d2 = d1 * d1;
+            if (st)
+                eval_out<PGH>(e, (long)ps, po, nf, val[0], PGH >= 2 ? val[1 % NO] * d1 : 0.0,
+                              PGH >= 2 ? val[2 % NO] * d1 : 0.0, PGH >= 3 ? val[3 % NO] * d2 : 0.0,
+                              PGH >= 3 ? val[4 % NO] * d2 : 0.0, PGH >= 3 ? val[5 % NO] * d2 : 0.0);
+        }
+    }
+}
+
+template <int NB, int PGH>
+static void eval2_top_launch(const Top2Args& a, const EvalArgs& e, hipStream_t s)
+{
+    const size_t lds = (size_t)8 * ((a.npw / 2 + 3) / 4) * 16 * (NB | 1) * sizeof(double) +
+                       a.nshift * sizeof(double2);
+    klaunch(KID_EVAL_TOP, k_eval2_top<NB, PGH>, dim3(a.grid), dim3(256), (unsigned)lds, s, a, e);
+}
+
+template <int NB>
+static void eval2_top_pgh(const Top2Args& a, const EvalArgs& e, hipStream_t s)
+{
+    if (e.ifpgh >= 3)
+        eval2_top_launch<NB, 3>(a, e, s);
+    else if (e.ifpgh == 2)
+        eval2_top_launch<NB, 2>(a, e, s);
+    else
+        eval2_top_launch<NB, 1>(a, e, s);
+}
+
+void launch_eval2_top(const Top2Args& a, const EvalArgs& e, hipStream_t s)
+{
+    if (a.ntop <= 0) return;
+    const int nb = (a.npw + 15) / 16;
+    if (a.npw < 2 || nb > 4) fail(-3, "2D plane-wave length above 64 on the whole-box route");
+    switch (nb) {
+    case 1: eval2_top_pgh<1>(a, e, s); break;
+    case 2: eval2_top_pgh<2>(a, e, s); break;
+    case 3: eval2_top_pgh<3>(a, e, s); break;
+    default: eval2_top_pgh<4>(a, e, s); break;
+    }
+}
+
+void launch_top_leaves2(const TopLeafArgs& a, hipStream_t s)
+{
+    top_leaves_launch<2>(a, s);
 }
 
 // ---------------------------------------------------------------------------

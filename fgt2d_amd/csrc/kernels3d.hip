@@ -18,6 +18,7 @@
 #include <mutex>
 
 #include "fgtpw_impl.hpp"
+#include "top_phase.hpp"
 
 namespace fgtpw {
 
@@ -2102,81 +2103,6 @@ void launch_pw_eval3(const Eval3Args& a, hipStream_t s)
 // sources with gradients, 2*10^4 targets with Hessians (npw 44, leaves of
 // order 34): 5690 -> 380 and 20700 -> 1930.
 // ---------------------------------------------------------------------------
-constexpr int TOP_RF = 66;  // 1/j!, j < TOP_RF
-struct TopFactorials {
-    double v[TOP_RF];
-    constexpr TopFactorials() : v()
-    {
-        double f = 1.0;
-        for (int j = 0; j < TOP_RF; ++j) {
-            if (j > 0) f *= j;
-            v[j] = 1.0 / f;
-        }
-    }
-};
-__constant__ const TopFactorials c_rf = TopFactorials();
-
-// one point alone; not inlined: the rare path must not cost the common one
-// its registers
-__device__ __noinline__ double2 top_series1(double u, int m)
-{
-    double c = 0, sn = 0;
-    if (m < 0) {
-        sincos(u, &sn, &c);
-        return make_double2(c, sn);
-    }
-    const double v = -u * u;
-    int k = (m - 1) >> 1;  // cosine terms 0..k, sine terms 0..k (k - 1 for odd m)
-    if (m & 1) {
-        c = c_rf.v[2 * k];
-        --k;
-    }
-    for (; k >= 0; --k) {
-        c = c * v + c_rf.v[2 * k];
-        sn = sn * v + c_rf.v[2 * k + 1];
-    }
-    return make_double2(c, sn * u);
-}
-
-// e[i] = sum_{j<m[i]} (i u[i])^j / j!; m[i] < 0: e^{i u[i]}.  U independent
-// Horner chains at once; where every m of the wavefront is the same (points of
-// one level) the factorials are scalar loads.
-template <int U>
-__device__ __forceinline__ void top_series(const double (&u)[U], const int (&m)[U], double2 (&e)[U])
-{
-    const int mu = __builtin_amdgcn_readfirstlane(m[0]);
-    bool same = true;
-#pragma unroll
-    for (int i = 0; i < U; ++i) same = same && m[i] == mu;
-    if (__all(same) && mu >= 0) {
-        double v[U];
-#pragma unroll
-        for (int i = 0; i < U; ++i) {
-            v[i] = -u[i] * u[i];
-            e[i] = make_double2(0.0, 0.0);
-        }
-        int k = (mu - 1) >> 1;
-        if (mu & 1) {
-#pragma unroll
-            for (int i = 0; i < U; ++i) e[i].x = c_rf.v[2 * k];
-            --k;
-        }
-        for (; k >= 0; --k) {
-            const double fc = c_rf.v[2 * k], fs = c_rf.v[2 * k + 1];
-#pragma unroll
-            for (int i = 0; i < U; ++i) {
-                e[i].x = e[i].x * v[i] + fc;
-                e[i].y = e[i].y * v[i] + fs;
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < U; ++i) e[i].y *= u[i];
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < U; ++i) e[i] = top_series1(u[i], m[i]);
-}
-
 // a point's leaf as the phase tables need it
 struct TopLeaf {
     double u[3];  // (x - c_leaf)/sqrt(delta)
@@ -2196,14 +2122,6 @@ __device__ __forceinline__ TopLeaf top_leaf(const Top3Args& a, long i, bool form
     L.m = form ? q.mf : q.me;
     return L;
 }
-
-// e times the shift
-__device__ __forceinline__ double2 top_shift(const double2 e, const double2 sh)
-{
-    return make_double2(e.x * sh.x - e.y * sh.y, e.x * sh.y + e.y * sh.x);
-}
-// m - k terms (the k-th derivative's), whole exponentials staying whole
-__device__ __forceinline__ int top_less(int m, int k) { return m < 0 ? m : max(m - k, 0); }
 
 // Formation.  One block of 4 wavefronts per (box, run of 4 TW column tiles):
 // rows (cos, sin) of the x nodes, columns (y node, z node, cos or sin of y, re
@@ -2313,7 +2231,7 @@ __global__ __launch_bounds__(256, NB <= 3 ? 2 : 1) void k_form3_top(Top3Args a)
             for (int sl0 = lsrc; sl0 < 4 * nks; sl0 += U * nsrc) {
                 double u[U];
                 int m[U];
-                double2 sh[U], e[U], e1[U];
+                double2 sh[U], es[DIP ? 2 : 1][U];
 #pragma unroll
                 for (int i = 0; i < U; ++i) {
                     const int sl = sl0 + i * nsrc;
@@ -2321,21 +2239,17 @@ __global__ __launch_bounds__(256, NB <= 3 ? 2 : 1) void k_form3_top(Top3Args a)
                     m[i] = irec[4 * sl + 3];
                     sh[i] = shl[irec[4 * sl + ax] + node];
                 }
-                top_series<U>(u, m, e);
-                if (DIP) {
-                    // (C', S') = ts (-S, C) of one term fewer
-#pragma unroll
-                    for (int i = 0; i < U; ++i) m[i] = top_less(m[i], 1);
-                    top_series<U>(u, m, e1);
-                }
+                top_series<U, DIP ? 2 : 1>(u, m, es);
+                double2 e[U], e1[U];
 #pragma unroll
                 for (int i = 0; i < U; ++i) {
                     const int sl = sl0 + i * nsrc;
-                    e[i] = top_shift(e[i], sh[i]);
+                    e[i] = top_shift(es[0][i], sh[i]);
                     e[i].x *= wsn;
                     e[i].y *= wsn;
                     if (DIP) {
-                        const double2 g = top_shift(e1[i], sh[i]);
+                        // (C', S') = ts (-S, C) of one term fewer
+                        const double2 g = top_shift(es[DIP ? 1 : 0][i], sh[i]);
                         e1[i] = make_double2(-tsn * wsn * g.y, tsn * wsn * g.x);
                     }
                     if (ax == 0) {
@@ -2543,22 +2457,21 @@ __global__ __launch_bounds__(256, PGH == 1 && NB <= 2 ? 3 : (PGH < 3 && NB <= 3 
         for (int k0 = 0; k0 < KS; k0 += 4) {
             double u[4], tsk[4];
             int m[4];
-            double2 sh[4], e[4];
+            double2 sh[4], e[NX][4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
+                m[q] = L.m;
                 const int node = min((4 * (k0 + q) + k4) >> 1, half - 1);
                 tsk[q] = a.ts[node];
                 sh[q] = a.shift[L.row[0] + node];
                 u[q] = tsk[q] * L.u[0];
             }
+            top_series<4, NX>(u, m, e);
 #pragma unroll
             for (int d = 0; d < NX; ++d) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) m[q] = top_less(L.m, d);
-                top_series<4>(u, m, e);
-#pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const double2 f = top_shift(e[q], sh[q]);
+                    const double2 f = top_shift(e[d][q], sh[q]);
                     const bool sn = k4 & 1;
                     const double x = d == 0 ? (sn ? f.y : f.x)
                                             : (d == 1 ? tsk[q] * (sn ? f.x : -f.y)
@@ -2577,22 +2490,35 @@ __global__ __launch_bounds__(256, PGH == 1 && NB <= 2 ? 3 : (PGH < 3 && NB <= 3 
         __syncthreads();  // the zeros; the last segment's readers are done
         stage(slab);
         __syncthreads();
+        // z series of four nodes at a time where the registers allow it
+        constexpr int ZB = NB >= 3 ? 4 : 1;
+        double2 zb[ZB];
         for (int c = 0; c < half; ++c) {
             if (c + 1 < half) load(c + 1);
             if (act) {
                 // z factors: lane (point i16, derivative k4), fetched per row
-                double vc, vs;
-                {
-                    const double tsn = a.ts[c];
-                    const int dz = PGH == 1 ? 0 : min(k4, PGH - 1);
-                    const double u[1] = {tsn * L.u[2]};
-                    const int m[1] = {top_less(L.m, dz)};
-                    double2 e1[1];
-                    top_series<1>(u, m, e1);
-                    const double2 e = top_shift(e1[0], a.shift[L.row[2] + c]);
-                    vc = dz == 0 ? e.x : (dz == 1 ? -tsn * e.y : -tsn * tsn * e.x);
-                    vs = dz == 0 ? e.y : (dz == 1 ? tsn * e.x : -tsn * tsn * e.y);
+                const int dz = PGH == 1 ? 0 : min(k4, PGH - 1);
+                const double tsc = a.ts[c];
+                if (c % ZB == 0) {
+                    double u[ZB];
+                    int m[ZB];
+                    double2 es[1][ZB];
+#pragma unroll
+                    for (int q = 0; q < ZB; ++q) {
+                        u[q] = a.ts[min(c + q, half - 1)] * L.u[2];
+                        m[q] = top_less(L.m, dz);
+                    }
+                    top_series<ZB, 1>(u, m, es);
+#pragma unroll
+                    for (int q = 0; q < ZB; ++q)
+                        zb[q] = top_shift(es[0][q], a.shift[L.row[2] + min(c + q, half - 1)]);
                 }
+                double2 e = zb[0];
+#pragma unroll
+                for (int q = 1; q < ZB; ++q)
+                    if (c % ZB == q) e = zb[q];
+                const double vc = dz == 0 ? e.x : (dz == 1 ? -tsc * e.y : -tsc * tsc * e.x);
+                const double vs = dz == 0 ? e.y : (dz == 1 ? tsc * e.x : -tsc * tsc * e.y);
                 const double2* sl = (const double2*)(slab + (c & 1) * sstride) + k4 * CS + i16;
 #pragma unroll
                 for (int nt = 0; nt < NB; ++nt) {
@@ -2649,22 +2575,20 @@ __global__ __launch_bounds__(256, PGH == 1 && NB <= 2 ? 3 : (PGH < 3 && NB <= 3 
             const int col = 16 * nt + i16, node = min(col >> 1, half - 1);
             const double tsn = a.ts[node];
             double u[4], y[PGH][4];
-            int m0[4], m[4];
-            double2 sh[4], e[4];
+            int m[4];
+            double2 sh[4], e[PGH][4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 u[r] = tsn * __shfl(L.u[1], k4 + 4 * r, 64);
                 sh[r] = a.shift[__shfl(L.row[1], k4 + 4 * r, 64) + node];
-                m0[r] = __shfl(L.m, k4 + 4 * r, 64);
+                m[r] = __shfl(L.m, k4 + 4 * r, 64);
             }
+            top_series<4, PGH>(u, m, e);
 #pragma unroll
             for (int d = 0; d < PGH; ++d) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) m[r] = top_less(m0[r], d);
-                top_series<4>(u, m, e);
-#pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const double2 f = top_shift(e[r], sh[r]);
+                    const double2 f = top_shift(e[d][r], sh[r]);
                     const bool sn = col & 1;
                     y[d][r] = col < npw ? (d == 0 ? (sn ? f.y : f.x)
                                                   : (d == 1 ? tsn * (sn ? f.x : -f.y)
@@ -2771,51 +2695,9 @@ void launch_eval3_top(const Top3Args& a, hipStream_t s)
     }
 }
 
-// The leaf rank of every sorted point and the leaves' records: a wavefront
-// per leaf.
-__global__ __launch_bounds__(256) void k_top_leaves(Top3Args a, const int* __restrict__ ls,
-                                                    const int* __restrict__ ls2, int nleaves,
-                                                    const int* __restrict__ leaf_of_rank,
-                                                    const int* __restrict__ lev,
-                                                    const int* __restrict__ par,
-                                                    int* __restrict__ pb, int* __restrict__ pb2,
-                                                    TopRec* __restrict__ rec)
+void launch_top_leaves(const TopLeafArgs& a, hipStream_t s)
 {
-    const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (r >= nleaves) return;
-    const int b = leaf_of_rank[r], l = lev[b], d = l - a.ltop;
-    if (d < 0) return;  // above the cutoff level: no expansions
-    const int s0 = ls[r], s1 = ls[r + 1], t0 = ls2 ? ls2[r] : 0, t1 = ls2 ? ls2[r + 1] : 0;
-    for (int i = s0 + lane; i < s1; i += 64) pb[i] = r;
-    if (pb2)
-        for (int i = t0 + lane; i < t1; i += 64) pb2[i] = r;
-    if (lane != 0) return;
-    int top = b;
-    for (int k = 0; k < d; ++k) top = par[top];
-    TopRec q;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        q.c[k] = a.cen[3 * (long)b + k];
-        // the leaf's place among the 2^d boxes of its level along the axis
-        const int pos = (int)rint((q.c[k] - a.cen[3 * (long)top + k]) * a.ib[l] +
-                                  0.5 * ((1 << d) - 1));
-        q.row[k] = ((1 << d) - 1 + pos) * (a.npw / 2);
-    }
-    // plane-wave route: formation up to thresh sources, evaluation below
-    // thresh points
-    const int th = a.thresh[l], n = s1 - s0;
-    q.mf = th > 0 && (th == INT_MAX || n <= th) ? -1 : a.m[l];
-    q.me = th > 0 && (th == INT_MAX || n + (t1 - t0) < th) ? -1 : a.m[l];
-    rec[r] = q;
-}
-
-void launch_top_leaves(const Top3Args& a, const int* ls, const int* ls2, int nleaves,
-                       const int* leaf_of_rank, const int* lev, const int* par, int* pb, int* pb2,
-                       TopRec* rec, hipStream_t s)
-{
-    if (nleaves <= 0) return;
-    k_top_leaves<<<(nleaves + 3) / 4, 256, 0, s>>>(a, ls, ls2, nleaves, leaf_of_rank, lev, par, pb,
-                                                   pb2, rec);
+    top_leaves_launch<3>(a, s);
 }
 
 // ---------------------------------------------------------------------------
