@@ -1054,20 +1054,20 @@ void zero_outputs(const Call& q, int dim, hipStream_t s)
 // with delta 1e-4, eps 1e-6 (boxes of up to 7000): 0.40 -> 0.59 ms, by leaves.
 // FP64 only, and series of at most TOP_RF terms.
 bool top_route2(const std::vector<LeafRun>& leaves, const Call& q, int ltop, int npwlevel,
-                int nlevels, const std::vector<double>& bsz, int* most)
+                int nlevels, double bs0, const std::vector<int>& herm, int* most)
 {
     if (nlevels - ltop > TOP_DEPTH || nlevels >= TOP_LEVELS) return false;
     const int nadd = (q.rn ? 1 : 0) + std::max(q.ifpgh, q.ifpghtarg);
     double pmax = 0;
     int npw = 0;
-    planewave_terms(2 * bsz[0] / std::pow(2.0, ltop), q.delta, nadd > 2 ? q.eps / 100 : q.eps, &pmax,
+    planewave_terms(2 * bs0 / std::pow(2.0, ltop), q.delta, nadd > 2 ? q.eps / 100 : q.eps, &pmax,
                     &npw);
     if (npw < 2 || npw > 64) return false;
     const double n2 = (double)npw * npw;
     double cost[TOP_LEVELS], point[TOP_LEVELS];
     int ntm = 0;
     for (int l = ltop; l <= nlevels; ++l) {
-        int m = hermite_terms(2, bsz[l], q.delta, q.eps) + 1;
+        int m = herm[l] + 1;
         if (q.rn || q.ifpgh >= 2 || q.ifpghtarg >= 2) m += nadd;
         ntm = std::max(ntm, m - 1);
         if (l >= std::max(npwlevel + 1, 0) && m > TOP_RF) return false;
@@ -1144,10 +1144,12 @@ void run2d(Workspace& W, const Call& q, hipStream_t s)
     // deepest level: first whose Hermite length is <= 18 (fgt2d.f:175-186)
     const int nlevstart = std::max(npwlevel, 0);
     int nlmax = npwlevel + 4;
+    std::vector<int> herm(nlevstart, 0);  // Hermite length per level, kept for the steps below
     {
         double bsize = bs0 / (double)(1 << nlevstart);
         for (int i = nlevstart; i <= 100; ++i) {
-            if (hermite_terms(2, bsize, q.delta, q.eps) <= 18) {
+            herm.push_back(hermite_terms(2, bsize, q.delta, q.eps));
+            if (herm.back() <= 18) {
                 nlmax = i;
                 break;
             }
@@ -1312,7 +1314,7 @@ void run2d(Workspace& W, const Call& q, hipStream_t s)
     bsz0[0] = bs0;
     for (int l = 0; l < L0; ++l) bsz0[l + 1] = bsz0[l] / 2;  // as the builder halves
     int most = 0;
-    const bool top0 = npwlevel < L0 && top_route2(leaves, q, nlevstart, npwlevel, L0, bsz0, &most);
+    const bool top0 = npwlevel < L0 && top_route2(leaves, q, nlevstart, npwlevel, L0, bs0, herm, &most);
     const bool early_ok = !g_serial && !tm.on && !W.arena && npwlevel < L0 && L0 >= 1 &&
                           L0 >= std::max(npwlevel + 1, 0) && !top0;
     struct Early {
@@ -1371,7 +1373,7 @@ void run2d(Workspace& W, const Call& q, hipStream_t s)
             const int npg0 = std::max(q.ifpgh, q.ifpghtarg), nadd0 = ifdipole + npg0;
             int ntm = 0, nlL = 0;
             for (int i = std::max(npwlevel, 0); i <= L; ++i) {
-                int nl = hermite_terms(2, bsz0[i], q.delta, q.eps);
+                int nl = herm[i];
                 if (ifdipole || q.ifpgh >= 2 || q.ifpghtarg >= 2) nl += nadd0;
                 ntm = std::max(ntm, nl);
                 if (i == L) nlL = nl;
@@ -1440,7 +1442,7 @@ void run2d(Workspace& W, const Call& q, hipStream_t s)
     std::vector<int> nlocal(nlevels + 1, 0);
     int ntermmax = 0;
     for (int i = nlevstart; i <= nlevels; ++i) {
-        nlocal[i] = hermite_terms(2, T.bsz[i], q.delta, q.eps);
+        nlocal[i] = herm[i];
         if (ifdipole || q.ifpgh >= 2 || q.ifpghtarg >= 2) nlocal[i] += nadd;
         ntermmax = std::max(ntermmax, nlocal[i]);
     }
@@ -2384,10 +2386,12 @@ void run3d(Workspace& W, const Call& q, hipStream_t s)
     }
     const int nlevstart = std::max(npwlevel, 0);
     int nlmax = npwlevel + 4;
+    std::vector<int> herm(nlevstart, 0);  // Hermite length per level, kept for the steps below
     {
         double bsize = bs0 / (double)(1 << nlevstart);
         for (int i = nlevstart; i <= 100; ++i) {
-            if (hermite_terms(3, bsize, q.delta, q.eps) <= 15) {
+            herm.push_back(hermite_terms(3, bsize, q.delta, q.eps));
+            if (herm.back() <= 15) {
                 nlmax = i;
                 break;
             }
@@ -2513,7 +2517,7 @@ void run3d(Workspace& W, const Call& q, hipStream_t s)
     std::vector<int> nlocal(nlevels + 1, 0);
     int ntermmax = 0;
     for (int i = nlevstart; i <= nlevels; ++i) {
-        nlocal[i] = hermite_terms(3, T.bsz[i], q.delta, q.eps);
+        nlocal[i] = herm[i];
         if (ifdipole || q.ifpgh >= 2 || q.ifpghtarg >= 2) nlocal[i] += nadd;
         ntermmax = std::max(ntermmax, nlocal[i]);
     }
