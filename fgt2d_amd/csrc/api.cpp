@@ -1461,8 +1461,9 @@ void run2d(Workspace& W, const Call& q, hipStream_t s)
     const bool mixed = g_precision == 1 && expansions && q.eps >= kMixedEpsMin && ntermmax < 63;
     const size_t esz = mixed ? sizeof(float) : sizeof(double);
 
-    // the cutoff-level boxes formed and evaluated whole (k_form2_top, k_eval2_top)
-    const bool top = top0 && expansions && nlevels == L0;
+    // the cutoff-level boxes formed and evaluated whole (k_form2_top, k_eval2_top);
+    // not if another thread has changed the arithmetic since the estimate
+    const bool top = top0 && expansions && nlevels == L0 && !mixed;
 
     // box arrays; expansion slots: the finest level first (its leaves are
     // formed first, possibly before the tree), then the other levels from
