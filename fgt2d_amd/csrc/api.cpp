@@ -2303,6 +2303,9 @@ bool top_route3(const std::vector<LeafRun>& leaves, const Call& q, int ltop, int
                 int nlevels, int npw, const std::vector<int>& nlocal)
 {
     if (nlevels - ltop > TOP_DEPTH || nlevels >= TOP_LEVELS) return false;
+    // no nodes (a small box at low accuracy): the expansions are empty, which
+    // the leaf kernels take and the whole-box ones do not
+    if (npw < 2) return false;
     const double n3 = (double)npw * npw * npw;
     // sources and leaves below the cutoff level, and the fullest box there
     double cost[TOP_LEVELS], m3[TOP_LEVELS];

@@ -3405,7 +3405,7 @@ void launch_form2_top(const Top2Args& a, hipStream_t s)
 {
     if (a.ntop <= 0) return;
     const int nb = (a.npw + 15) / 16;
-    if (a.npw < 2 || nb > 4) fail(-3, "2D plane-wave length above 64 on the whole-box route");
+    if (a.npw < 2 || nb > 4) fail(-3, "2D plane-wave length outside 2..64 on the whole-box route");
     const bool dip = a.dipw != nullptr;
     switch (nb) {
     case 1: dip ? form2_top_launch<1, true>(a, s) : form2_top_launch<1, false>(a, s); break;
@@ -3606,7 +3606,7 @@ void launch_eval2_top(const Top2Args& a, const EvalArgs& e, hipStream_t s)
 {
     if (a.ntop <= 0) return;
     const int nb = (a.npw + 15) / 16;
-    if (a.npw < 2 || nb > 4) fail(-3, "2D plane-wave length above 64 on the whole-box route");
+    if (a.npw < 2 || nb > 4) fail(-3, "2D plane-wave length outside 2..64 on the whole-box route");
     switch (nb) {
     case 1: eval2_top_pgh<1>(a, e, s); break;
     case 2: eval2_top_pgh<2>(a, e, s); break;

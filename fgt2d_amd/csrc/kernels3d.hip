@@ -2366,7 +2366,7 @@ void launch_form3_top(const Top3Args& a, hipStream_t s)
 {
     if (a.ntop <= 0) return;
     const int nb = (a.npw + 15) / 16;
-    if (a.npw < 2 || nb > 4) fail(-3, "3D plane-wave length above 64");
+    if (a.npw < 2 || nb > 4) fail(-3, "3D plane-wave length outside 2..64 on the whole-box route");
     const bool dip = a.dipw != nullptr;
     switch (nb) {
     case 1: dip ? form3_top_launch<1, true>(a, s) : form3_top_launch<1, false>(a, s); break;
@@ -2693,7 +2693,7 @@ void launch_eval3_top(const Top3Args& a, hipStream_t s)
 {
     if (a.ntop <= 0) return;
     const int nb = (a.npw + 15) / 16;
-    if (a.npw < 2 || nb > 4) fail(-3, "3D plane-wave length above 64");
+    if (a.npw < 2 || nb > 4) fail(-3, "3D plane-wave length outside 2..64 on the whole-box route");
     switch (nb) {
     case 1: eval3_top_pgh<1>(a, s); break;
     case 2: eval3_top_pgh<2>(a, s); break;

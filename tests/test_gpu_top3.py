@@ -71,3 +71,33 @@ def test_whole_box_route_matches_oracle(case):
         if (k < 3 and k < ifs) or (k >= 3 and k - 3 < ift):
             g, w = np.asarray(g), np.asarray(w)
             assert np.abs(g - w).max() < 1e-11 * np.abs(w).max(), NAMES[k]
+
+
+# (extent of the points, ns, nt, delta, eps, ifpgh, ifpghtarg, dipoles)
+FEW_NODES = [
+    (0.25, 500, 0, 1.0, 0.1, 1, 0, False),
+    (1.0, 900, 200, 6.9, 0.2, 2, 1, False),
+    (1.0, 600, 100, 6.9, 0.2, 1, 0, True),
+]
+
+
+@pytest.mark.parametrize("case", FEW_NODES, ids=[str(i) for i in range(len(FEW_NODES))])
+def test_no_plane_wave_nodes(case):
+    """Boxes so small and accuracies so low that the expansions have no node
+    at all: they add nothing, as in the oracle, and the call is no error."""
+    ext, ns, nt, delta, eps, ifs, ift, ifd = case
+    print("case", case, flush=True)
+    rng = np.random.default_rng(ns)
+    src, chg = ext * rng.random((ns, 3)), rng.normal(size=(ns, 1))
+    tg = ext * rng.random((nt, 3)) if nt else None
+    rn = rng.normal(size=(ns, 3)) if ifd else None
+    ds = rng.normal(size=(ns, 1)) if ifd else None
+    got = fgt2d_amd.fgt3d(delta, eps, src, chg, tg, ifpgh=ifs, ifpghtarg=ift, ifdipole=int(ifd),
+                          rnormal=rn, dipstr=ds)
+    st = fgt2d_amd.last_stats()
+    assert st["npw"] == 0 and st["nlevels"] > st["npwlevel"], st
+    want = O.oracle_fgt3d(delta, eps, src, chg, tg, ifpgh=ifs, ifpghtarg=ift, rnormal=rn,
+                          dipstr=ds)
+    for k, (g, w) in enumerate(zip(got, want)):
+        if (k < 3 and k < ifs) or (k >= 3 and k - 3 < ift):
+            assert np.array_equal(np.asarray(g), np.asarray(w)), NAMES[k]
