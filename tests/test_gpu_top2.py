@@ -63,16 +63,20 @@ def test_whole_box_route_matches_oracle(case):
 
 
 def test_mixed_arithmetic_stays_leaf_by_leaf():
+    """The same call, whole boxes in FP64 (third case above), by leaves in the
+    mixed mode, whose expansions are half as wide."""
     rng = np.random.default_rng(3)
-    src, chg = _pts.mixture(rng, 20000), rng.normal(size=(20000, 1))
-    prev = fgt2d_amd.set_precision("mixed")
-    fgt2d_amd.set_timing(True)
-    try:
-        got = fgt2d_amd.fgt2d(1e-4, 1e-6, src, chg)
-        kernels = {k["kernel"] for k in fgt2d_amd.kernel_launches()}
-        assert fgt2d_amd.last_precision() == "mixed" and "form_top" not in kernels
-    finally:
-        fgt2d_amd.set_timing(False)
-        fgt2d_amd.set_precision(prev)
-    want = O.oracle_fgt2d(1e-4, 1e-6, src, chg)
-    assert np.abs(got[0] - want[0]).max() < 2e-5 * np.abs(want[0]).max()
+    src, chg = _pts.uniform(rng, 30011), rng.normal(size=(30011, 1))
+    want = O.oracle_fgt2d(5e-4, 1e-6, src, chg)
+    for mode, whole, tol in (("fp64", True, 1e-11), ("mixed", False, 2e-5)):
+        prev = fgt2d_amd.set_precision(mode)
+        fgt2d_amd.set_timing(True)
+        try:
+            got = fgt2d_amd.fgt2d(5e-4, 1e-6, src, chg)
+            kernels = {k["kernel"] for k in fgt2d_amd.kernel_launches()}
+            assert fgt2d_amd.last_precision() == mode
+            assert ("form_top" in kernels) == whole and ("eval_top" in kernels) == whole, kernels
+        finally:
+            fgt2d_amd.set_timing(False)
+            fgt2d_amd.set_precision(prev)
+        assert np.abs(got[0] - want[0]).max() < tol * np.abs(want[0]).max()
