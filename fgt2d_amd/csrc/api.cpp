@@ -1039,6 +1039,16 @@ void zero_outputs(const Call& q, int dim, hipStream_t s)
     }
 }
 
+// FGTPW_ROUTE=leaves or boxes, read at every call: the route of a transform
+// that both can take (top_route2, top_route3), in place of the one estimated
+// faster; -1, 1, or 0 where it is not set
+int forced_route()
+{
+    const char* e = std::getenv("FGTPW_ROUTE");
+    if (!e) return 0;
+    return !std::strcmp(e, "leaves") ? -1 : (!std::strcmp(e, "boxes") ? 1 : 0);
+}
+
 // Route of a 2D transform with expansions: whole cutoff-level boxes at once
 // (k_form2_top, k_eval2_top) or leaf by leaf, whichever the estimate below
 // finds faster; *most: the sources of the fullest refined box.  As in 3D the
@@ -1096,6 +1106,7 @@ bool top_route2(const std::vector<LeafRun>& leaves, const Call& q, int ltop, int
     const double et = q.ifpghtarg > 0 ? (double)q.nt / q.ns : 0.0;
     const double form = std::max((0.1 + 8e-5 * n2) * nsum, (15 + 0.06 * n2) * *most) * (q.rn ? 2.5 : 1.0);
     const double eval = (0.1 + 1.3e-4 * n2) * nsum * (weight(q.ifpgh) + et * weight(q.ifpghtarg));
+    if (const int f = forced_route()) return f > 0;
     return form + eval < leafwise;  // every density costs the same again
 }
 
@@ -2343,6 +2354,7 @@ bool top_route3(const std::vector<LeafRun>& leaves, const Call& q, int ltop, int
     const double pt = 8e-5 * n3 + 0.2;
     const double form = pt * dip * std::max(nsum, 130.0 * most);
     const double eval = pt * nsum * (weight(q.ifpgh) + et * weight(q.ifpghtarg));
+    if (const int f = forced_route()) return f > 0;
     return form + eval < leafwise;  // every density costs the same again
 }
 
