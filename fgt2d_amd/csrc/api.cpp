@@ -2310,9 +2310,20 @@ void run_large_delta3(Workspace& W, const Call& q, hipStream_t s, int npwlevel, 
 // Measured (by leaves -> at once): 10^6 points, delta 1e-3, eps 1e-6 (23 a
 // leaf): 11.0 -> 4.8 ms; delta 3e-3 (111 a leaf): 2.8 -> 4.0 ms, so there by
 // leaves; 4*10^5, delta 3e-3, eps 1e-9 (21 a leaf): 22.4 -> 6.1 ms.
-bool top_route3(const std::vector<LeafRun>& leaves, const Call& q, int ltop, int npwlevel,
-                int nlevels, int npw, const std::vector<int>& nlocal)
+// The leaf records are the leaves before the level restriction.  A level of
+// order above 32 has few of them beside deeper neighbours, and the restriction
+// often refines every one: charging their kernels then put the estimate by
+// leaves up to 10 ms too high.  Such a level costs 0.2 npw^3 instead (its
+// sources' finer leaves; fit as above), if npw <= 48, where those run on
+// matrix cores, and if no leaf is left there that may hold targets.  1591
+// draws of clustered and uniform points, 10^3 to 2*10^5 of them: of 799 taken
+// at once 9 were slower than by leaves, by up to 1.7, then 2 of 789, by up to
+// 1.3; 27703 points in 10 clusters, delta 6.9e-3, eps 1e-9, with gradients:
+// 3.7 -> 2.0 ms.
+bool top_route3(const std::vector<LeafRun>& leaves, const Tree3D& T, const Call& q, int ltop,
+                int npwlevel, int npw, const std::vector<int>& nlocal)
 {
+    const int nlevels = T.nlevels;
     if (nlevels - ltop > TOP_DEPTH || nlevels >= TOP_LEVELS) return false;
     // no nodes (a small box at low accuracy): the expansions are empty, which
     // the leaf kernels take and the whole-box ones do not
@@ -2355,7 +2366,27 @@ bool top_route3(const std::vector<LeafRun>& leaves, const Call& q, int ltop, int
     const double form = pt * dip * std::max(nsum, 130.0 * most);
     const double eval = pt * nsum * (weight(q.ifpgh) + et * weight(q.ifpghtarg));
     if (const int f = forced_route()) return f > 0;
-    return form + eval < leafwise;  // every density costs the same again
+    // every density costs the same again
+    if (form + eval >= leafwise) return false;
+    auto is_leaf = [&](const LeafRun& r) {
+        int b = 0;
+        while (b >= 0 && T.nch[b] > 0 && T.lev[b] < r.level) {
+            const int* ch = &T.ch[8 * (size_t)b];
+            const uint64_t pre = r.key >> (3 * (r.level - T.lev[b] - 1));
+            b = -1;
+            for (int j = 0; j < 8; ++j)
+                if (ch[j] >= 0 && (uint64_t)T.pre[ch[j]] == pre) b = ch[j];
+        }
+        return b >= 0 && T.lev[b] == r.level && T.nch[b] == 0;
+    };
+    for (int l = ltop; l <= nlevels && npw <= 48; ++l) {
+        if (nlocal[l] + 1 <= 32 || count[l] == 0 || count[l] > 256) continue;
+        bool left = false;
+        for (int b = T.laddr[2 * l]; et > 0 && !left && b <= T.laddr[2 * l + 1]; ++b) left = T.nch[b] == 0;
+        for (size_t i = 0; !left && i < n; ++i) left = leaves[i].level == l && is_leaf(leaves[i]);
+        if (!left) leafwise -= (cost[l] - 0.2 * n3) * 256;
+    }
+    return form + eval < leafwise;
 }
 
 void run3d(Workspace& W, const Call& q, hipStream_t s)
@@ -2589,7 +2620,7 @@ void run3d(Workspace& W, const Call& q, hipStream_t s)
     std::vector<int> m2l_l;
     // the cutoff-level boxes formed and evaluated whole (k_form3_top, k_eval3_top)
     std::vector<int> tform_l, teval_l;
-    const bool top = expansions && top_route3(leaves, q, nlevstart, npwlevel, nlevels, npw, nlocal);
+    const bool top = expansions && top_route3(leaves, T, q, nlevstart, npwlevel, npw, nlocal);
     // chunks: upward (level of the formed leaves, first and last parent in
     // merge_l[level - 1], first and last leaf in form_l[level]); downward
     // (level, first and last box in eval_l[level])

@@ -6,8 +6,8 @@ plane-wave leaves, the chunks) are compared with the oracle also for the
 inputs that the route estimate gives to the whole-box kernels.
 
 Against each other: every form a call can have (plane-wave lengths 2 to 58,
-charges, dipoles or both, several densities, every pair of outputs, sparse and
-dense boxes, a single source, no targets) by leaves and by whole boxes.
+charges, dipoles or both, several densities, sources or targets alone,
+sparse and dense boxes, a single source) by leaves and by whole boxes.
 Tolerance: the same FP64 sums in another order, as the tests against the
 oracle."""
 import numpy as np
@@ -79,6 +79,7 @@ FORMS = [
     (2, "uniform", 901, 300, 2.1, 0.1, 1, 1, 1, True, False),      # npw 2, the root alone
     (2, "uniform", 2001, 501, 1.25, 0.02, 2, 1, 1, True, False),   # npw 4
     (2, "uniform", 2003, 33, 0.71, 1e-3, 1, 2, 0, True, False),    # npw 8
+    (2, "uniform", 1, 37, 0.71, 1e-3, 1, 0, 1, True, False),       # one source
     (2, "uniform", 5003, 1001, 1e-2, 1e-3, 1, 3, 3, True, True),
     (2, "cluster", 30001, 777, 1e-4, 1e-6, 2, 2, 1, False, True),  # thousands of points a box
     (2, "cluster", 20001, 0, 1e-4, 1e-9, 1, 3, 0, True, True),
@@ -87,6 +88,7 @@ FORMS = [
     (3, "uniform", 901, 300, 2.1, 0.1, 1, 1, 1, True, False),      # npw 2, the root alone
     (3, "uniform", 2001, 501, 1.25, 0.02, 2, 1, 1, True, False),   # npw 4
     (3, "uniform", 4003, 33, 0.71, 1e-3, 1, 2, 0, True, False),    # npw 8
+    (3, "uniform", 1, 37, 0.71, 1e-3, 1, 0, 1, True, False),       # one source
     (3, "uniform", 5003, 1001, 2e-2, 1e-3, 1, 3, 3, True, True),
     (3, "cluster", 30001, 777, 1e-3, 1e-6, 2, 2, 1, False, True),  # thousands of points a box
     (3, "cluster", 20001, 0, 1e-3, 1e-9, 1, 3, 0, True, True),

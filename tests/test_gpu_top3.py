@@ -32,6 +32,8 @@ CASES = [
     ("uniform", 5000, 400, 1e-2, 1e-12, 1, 2, 1, True, False, True),   # npw 52: the widest tiles
     ("uniform", 3000, 200, 2e-2, 1e-12, 1, 1, 2, True, False, True),
     ("uniform", 60000, 500, 1e-2, 1e-6, 1, 1, 1, True, False, False),  # full leaves: leaf by leaf
+    # its few leaves of order 33 are all refined by the level restriction
+    ("mixture", 27703, 0, 7e-3, 1e-9, 1, 2, 0, True, False, False),
 ]
 
 
@@ -40,6 +42,9 @@ def _points(kind, rng, n):
         return rng.random((n, 3))
     if kind == "cluster":
         return 0.485 + 0.03 * rng.random((n, 3))
+    if kind == "mixture":
+        mu = rng.uniform(0.1, 0.9, (10, 3))
+        return np.clip(mu[rng.integers(0, 10, n)] + 0.01 * rng.normal(size=(n, 3)), 0.0, 1.0)
     d = rng.normal(size=(n, 3))
     d /= np.linalg.norm(d, axis=1, keepdims=True)
     return 0.5 + d * (0.4 + 1e-3 * rng.normal(size=(n, 1)))
