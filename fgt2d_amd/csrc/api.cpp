@@ -1113,6 +1113,7 @@ bool top_route2(const std::vector<LeafRun>& leaves, const Call& q, int ltop, int
 void run2d(Workspace& W, const Call& q, hipStream_t s)
 {
     t_mixed = false;
+    W.last_valid = false;  // until this call's tree is built
     W.n_order = 0;
     Timer tm(W, s);
     const int ns = q.ns, nt = q.nt, nd = q.nd;
@@ -1436,7 +1437,6 @@ void run2d(Workspace& W, const Call& q, hipStream_t s)
 
     // ---------------- host: tree, lists, tables ----------------
     auto th0 = std::chrono::steady_clock::now();
-    W.last_valid = false;
     Tree2D& T = W.last;
     build_tree2d(T, leaves, nlmax, npwlevel, bs0, cen0);
     tm.build_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - th0).count();
@@ -2392,6 +2392,7 @@ bool top_route3(const std::vector<LeafRun>& leaves, const Tree3D& T, const Call&
 void run3d(Workspace& W, const Call& q, hipStream_t s)
 {
     t_mixed = false;
+    W.last_valid = false;  // until this call's tree is built
     if (!q.chg && !q.rn) {
         zero_outputs(q, 3, s);
         return;
@@ -2427,7 +2428,6 @@ void run3d(Workspace& W, const Call& q, hipStream_t s)
         npwlevel = -1000;
     }
     if (npwlevel < -2) {
-        W.last_valid = false;
         run_large_delta3(W, q, s, npwlevel, bs0, cen0, tm);
         return;
     }
@@ -2551,7 +2551,6 @@ void run3d(Workspace& W, const Call& q, hipStream_t s)
 
     // ---------------- host: tree, lists, tables ----------------
     auto th0 = std::chrono::steady_clock::now();
-    W.last_valid = false;
     Tree3D& T = W.last3;
     build_tree<3>(T, leaves, nlmax, npwlevel, bs0, cen0);
     tm.build_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - th0).count();

@@ -159,6 +159,22 @@ def test_invalid_arguments_are_rejected():
     fgt2d_amd.fgt2d(1e-3, 1e-6, src, chg, None, ifpgh=1)
 
 
+def test_no_tree_after_a_call_without_one():
+    """The large-delta branch builds no tree: asking for the last one is an
+    error then, not an earlier call's tree."""
+    rng = np.random.default_rng(2)
+    for dim, f, tree in ((2, fgt2d_amd.fgt2d, fgt2d_amd.last_tree2d),
+                         (3, fgt2d_amd.fgt3d, fgt2d_amd.last_tree3d)):
+        src = rng.random((3000, dim))
+        chg = np.ones((3000, 1))
+        f(1e-2, 1e-3, src, chg)
+        assert tree(3000, 0)["nboxes"] > 1
+        f(50.0, 1e-3, src, chg)
+        with pytest.raises(fgt2d_amd.FGTError) as e:
+            tree(3000, 0)
+        assert e.value.code == fgt2d_amd.FGTPW_EINVAL, dim
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_finest_level_formed_beside_the_tree_is_bit_identical(precision):
     """The finest level's leaves are formed while the host builds the tree
