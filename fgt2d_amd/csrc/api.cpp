@@ -1062,6 +1062,12 @@ int forced_route()
 // them (119 a leaf): 0.89 -> 1.00 ms, so there by leaves; 10^6 with gradients,
 // delta 6.8e-6, eps 5e-11 (orders above 32): 4.5 -> 2.1 ms; 10^5 mixture points
 // with delta 1e-4, eps 1e-6 (boxes of up to 7000): 0.40 -> 0.59 ms, by leaves.
+// A box's serial sum takes 39 to 45 ns a source up to npw 32 (57 to 70 with
+// dipoles), however few nodes: charged at 45 and 50, a tenth more for the
+// launch.  Without that floor (3442 draws, 10^3 to 1.6*10^6 points) 50 of 1301
+// calls taken at once were more than 5% slower than by leaves, by up to 1.32
+// (25401 uniform points, eps 1e-3, gradients at 2198 targets, 2857 sources a
+// box: 0.28 -> 0.36 ms); with it 18 of 1218, by up to 1.22.
 // FP64 only, and series of at most TOP_RF terms.
 bool top_route2(const std::vector<LeafRun>& leaves, const Call& q, int ltop, int npwlevel,
                 int nlevels, double bs0, const std::vector<int>& herm, int* most)
@@ -1104,7 +1110,9 @@ bool top_route2(const std::vector<LeafRun>& leaves, const Call& q, int ltop, int
     auto weight = [](int ifpgh) { return ifpgh <= 0 ? 0.0 : (ifpgh == 1 ? 1.0 : (ifpgh == 2 ? 3.0 : 6.0)); };
     // evaluated points as if spread like the sources
     const double et = q.ifpghtarg > 0 ? (double)q.nt / q.ns : 0.0;
-    const double form = std::max((0.1 + 8e-5 * n2) * nsum, (15 + 0.06 * n2) * *most) * (q.rn ? 2.5 : 1.0);
+    const double form = std::max(
+        std::max((0.1 + 8e-5 * n2) * nsum, (15 + 0.06 * n2) * *most) * (q.rn ? 2.5 : 1.0),
+        (npw <= 16 ? 45 : 50) * (q.rn ? 1.6 : 1.0) * *most);
     const double eval = (0.1 + 1.3e-4 * n2) * nsum * (weight(q.ifpgh) + et * weight(q.ifpghtarg));
     if (const int f = forced_route()) return f > 0;
     return form + eval < leafwise;  // every density costs the same again

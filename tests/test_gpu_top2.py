@@ -30,6 +30,8 @@ CASES = [
     ("uniform", 60013, 501, 3e-4, 1e-9, 1, 3, 1, True, False, True),     # npw 44
     ("uniform", 8000, 2000, 1e-3, 1e-12, 1, 1, 2, True, False, True),    # npw 52: the widest tiles
     ("uniform", 200000, 1000, 1e-2, 1e-6, 1, 1, 1, True, False, False),  # full leaves: leaf by leaf
+    # thousands of sources a box and 12 nodes: the serial sum is the longer
+    ("uniform", 25401, 2198, 1.6e-2, 1e-3, 1, 0, 2, True, False, False),
 ]
 
 
