@@ -928,8 +928,8 @@ const Tables3D& tables3d(Workspace& W, int npw, double pmax, int ntermmax, int n
                          double xm, bool leafwise, hipStream_t s)
 {
     Tables3D& t = W.tab3;
-    if (t.valid && (t.leafwise || !leafwise) && t.npw == npw && t.pmax == pmax && t.ntermmax == ntermmax && t.nmax == nmax &&
-        t.xmin2 == xmin2 && t.xm == xm)
+    if (t.valid && (t.leafwise || !leafwise) && t.npw == npw && t.pmax == pmax &&
+        t.ntermmax == ntermmax && t.nmax == nmax && t.xmin2 == xmin2 && t.xm == xm)
         return t;
     const int half = npw / 2, mt = ntermmax + 1;
     const size_t nexp = (size_t)npw * npw * half;
@@ -1059,9 +1059,9 @@ int forced_route()
 // routes over uniform and mixture points, 3*10^3 to 2*10^6 of them, delta
 // 1e-5..1e-2, eps 1e-3, 1e-6, 1e-9.  Measured (by leaves -> at once): 10^5
 // uniform points, delta 1e-4, eps 1e-9 (47 a leaf): 0.46 -> 0.38 ms, 10^6 of
-// them (119 a leaf): 0.89 -> 1.00 ms, so there by leaves; 10^6 with gradients,
-// delta 6.8e-6, eps 5e-11 (orders above 32): 4.5 -> 2.1 ms; 10^5 mixture points
-// with delta 1e-4, eps 1e-6 (boxes of up to 7000): 0.40 -> 0.59 ms, by leaves.
+// them (119 a leaf): 0.89 -> 1.10 ms, so there by leaves; 10^6 with gradients,
+// delta 6.8e-6, eps 5e-11 (orders above 32): 4.5 -> 2.2 ms; 10^5 mixture points
+// with delta 1e-4, eps 1e-6 (boxes of up to 7000): 0.37 -> 0.65 ms, by leaves.
 // A box's serial sum takes 39 to 45 ns a source up to npw 32 (57 to 70 with
 // dipoles), however few nodes: charged at 45 and 50, a tenth more for the
 // launch.  Without that floor (3442 draws, 10^3 to 1.6*10^6 points) 50 of 1301
@@ -2316,8 +2316,8 @@ void run_large_delta3(Workspace& W, const Call& q, hipStream_t s, int npwlevel, 
 //              order <= 32, 0.44 npw^3 above (kernels without matrix cores),
 //              1.5e-4 m^3 a point and side; 30 us of more launches.
 // Measured (by leaves -> at once): 10^6 points, delta 1e-3, eps 1e-6 (23 a
-// leaf): 11.0 -> 4.8 ms; delta 3e-3 (111 a leaf): 2.8 -> 4.0 ms, so there by
-// leaves; 4*10^5, delta 3e-3, eps 1e-9 (21 a leaf): 22.4 -> 6.1 ms.
+// leaf): 10.9 -> 4.9 ms; delta 3e-3 (111 a leaf): 2.8 -> 4.1 ms, so there by
+// leaves; 4*10^5, delta 3e-3, eps 1e-9 (21 a leaf): 22.3 -> 6.0 ms.
 // The leaf records are the leaves before the level restriction.  A level of
 // order above 32 has few of them beside deeper neighbours, and the restriction
 // often refines every one: charging their kernels then put the estimate by
@@ -2390,7 +2390,8 @@ bool top_route3(const std::vector<LeafRun>& leaves, const Tree3D& T, const Call&
     for (int l = ltop; l <= nlevels && npw <= 48; ++l) {
         if (nlocal[l] + 1 <= 32 || count[l] == 0 || count[l] > 256) continue;
         bool left = false;
-        for (int b = T.laddr[2 * l]; et > 0 && !left && b <= T.laddr[2 * l + 1]; ++b) left = T.nch[b] == 0;
+        for (int b = T.laddr[2 * l]; et > 0 && !left && b <= T.laddr[2 * l + 1]; ++b)
+            left = T.nch[b] == 0;
         for (size_t i = 0; !left && i < n; ++i) left = leaves[i].level == l && is_leaf(leaves[i]);
         if (!left) leafwise -= (cost[l] - 0.2 * n3) * 256;
     }
@@ -2959,7 +2960,6 @@ void run3d(Workspace& W, const Call& q, hipStream_t s)
         if (use_src) L.l[L.count++] = SegList{d_teval, (int)nte, src_se, 64, seg_s, box_s};
         launch_seg_scan(L, s);
         Top3Args ta{};
-        ta.cen = d_cen;
         ta.rec = rec;
         ta.nd = nd;
         ta.dsq = dsq;

@@ -331,7 +331,7 @@ struct Top2Args {
     // evaluation: segments of TOP2_SEG points (as SegList), outputs as EvalArgs
     const int *tstart, *segbox;
     int grid;
-    int waves;              // formation: wavefronts per box, 1 to 8
+    int waves;              // formation: wavefronts per box, 4 or 8
 };
 constexpr int TOP2_SEG = 256;
 void launch_top_leaves2(const TopLeafArgs& a, hipStream_t s);
@@ -413,7 +413,6 @@ void launch_form3_pw(const Form3Args& a, hipStream_t s);
 struct Top3Args {
     const int* tops;        // cutoff-level boxes
     int ntop;
-    const double* cen;      // 3 per box
     const int2* se;         // point ranges of the boxes (sources, or the evaluated points)
     const int* pbox;        // leaf rank of every sorted point
     const TopRec* rec;      // per leaf rank

@@ -3234,11 +3234,12 @@ __device__ __forceinline__ void pair_add(double dx, double dy, double q, double 
 // the pair of one node and supplies the cosine to one 16-wide tile and the
 // sine to the next (nodes in groups of 16; a last group of at most 8 shares
 // one tile, cosines in lanes 0-7, sines in 8-15).  Bound by the series (FP64
-// VALU) and latency; the matrix pipe is 20-25% busy.  Against the leaf kernels
-// they replace, us: 10^6 uniform points with gradients, eps 5e-11 (npw 44,
-// leaves of order 37 and 24): formation and merge 1600 -> 335, conversion,
-// split and evaluation 2250 -> 800; 10^5, eps 1e-9 (npw 38): 120 -> 42 and
-// 86 -> 46.
+// VALU) and latency; the matrix pipe is busy for 21% of the formation and 16% of
+// the evaluation at 10^6 points with gradients, 13% and 5% at 10^5.  Against the
+// leaf kernels they replace, us: 10^6 uniform points with gradients, eps 5e-11
+// (npw 44, leaves of order 37 and 24): formation and merge 1600 -> 315,
+// conversion, split and evaluation 2250 -> 810; 10^5, eps 1e-9 (npw 38): 120 ->
+// 43 and 86 -> 48.
 // ---------------------------------------------------------------------------
 // place of (node, sine or cosine) among the 16 NB rows or columns
 template <int NB>
@@ -3255,7 +3256,7 @@ __device__ __forceinline__ int top2_node(int g, int i16)
     return (NB & 1) && g == NB / 2 ? 16 * g + (i16 & 7) : 16 * g + i16;
 }
 
-// Formation: one block of 2 to 8 wavefronts per (box, density), which take
+// Formation: one block of 4 or 8 wavefronts per (box, density), which take
 // groups of 4 sources in turn through the MFMA K dimension, and the
 // wavefronts' sums are added in order.  With dipoles the product gains
 // X (w2 Y') + X' (w1 Y), primes the derivatives along the axis.

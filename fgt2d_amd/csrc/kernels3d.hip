@@ -18,7 +18,6 @@
 #include <mutex>
 
 #include "fgtpw_impl.hpp"
-#include "near_stage.hpp"
 #include "top_phase.hpp"
 
 namespace fgtpw {
@@ -2102,13 +2101,17 @@ void launch_pw_eval3(const Eval3Args& a, hipStream_t s)
 // point, on FP64 matrix cores.  No leaf expansion is formed, stored, merged,
 // split or converted; the values differ from the leaf-by-leaf route by
 // rounding alone (2-norm 1e-15).
-// Bound by the FP64 matrix pipe (64 cycles an MFMA, about 40% busy), behind
-// it the phase tables and barriers.  Against the leaf kernels they replace,
-// us: 10^6 uniform points, eps 1e-6 (npw 26): formation and merge 4500 ->
-// 1420, conversion, split and evaluation 4270 -> 1420; 8M shell sources + 8M
-// targets, eps 1e-9 (npw 38): 126000 -> 34000 and 158000 -> 15000; 5*10^4
-// sources with gradients, 2*10^4 targets with Hessians (npw 44, leaves of
-// order 34): 5690 -> 380 and 20700 -> 1930.
+// Bound by latency: the matrix pipe is busy for 37 to 42% of the time (npw 26;
+// formation at npw 38 as well), 28% in the evaluation at npw 38 and 17 to 26%
+// with derivatives at npw 44; the rest is the phase series on the VALU, the
+// staging, barriers and scratch traffic in the instances held to two or three
+// wavefronts per SIMD (spilled registers: evaluation of values 29 up to npw 32,
+// 84 up to 48, 122 with gradients; formation above npw 32 46, 193 with dipoles).
+// Against the leaf kernels they replace, us: 10^6 uniform points, eps 1e-6 (npw 26):
+// formation and merge 4500 -> 1530, conversion, split and evaluation 4270 ->
+// 1510; 8M shell sources + 8M targets, eps 1e-9 (npw 38): 126000 -> 34500 and
+// 158000 -> 12000; 5*10^4 sources with gradients, 2*10^4 targets with Hessians
+// (npw 44, leaves of order 34): 5690 -> 410 and 20700 -> 1820.
 // ---------------------------------------------------------------------------
 // a point's leaf as the phase tables need it
 struct TopLeaf {
@@ -2117,7 +2120,8 @@ struct TopLeaf {
     int m;        // terms; -1: whole exponentials
 };
 
-__device__ __forceinline__ TopLeaf top_leaf(const Top3Args& a, long i, bool form)
+// the evaluated point i's
+__device__ __forceinline__ TopLeaf top_leaf(const Top3Args& a, long i)
 {
     TopLeaf L;
     const TopRec q = a.rec[a.pbox[i]];
@@ -2126,7 +2130,7 @@ __device__ __forceinline__ TopLeaf top_leaf(const Top3Args& a, long i, bool form
         L.u[k] = (a.pts[3 * i + k] - q.c[k]) * a.dsq;
         L.row[k] = q.row[k];
     }
-    L.m = form ? q.mf : q.me;
+    L.m = q.me;
     return L;
 }
 
@@ -2459,7 +2463,7 @@ __global__ __launch_bounds__(256, PGH == 1 && NB <= 2 ? 3 : (PGH < 3 && NB <= 3 
         };
         load(0);
         double X[NX][KS], acc[NA][NB][4];
-        const TopLeaf L = top_leaf(a, min(t0 + i16, p1 - 1), false);
+        const TopLeaf L = top_leaf(a, min(t0 + i16, p1 - 1));
 #pragma unroll
         for (int k0 = 0; k0 < KS; k0 += 4) {
             double u[4], tsk[4];
@@ -2497,7 +2501,9 @@ __global__ __launch_bounds__(256, PGH == 1 && NB <= 2 ? 3 : (PGH < 3 && NB <= 3 
         __syncthreads();  // the zeros; the last segment's readers are done
         stage(slab);
         __syncthreads();
-        // z series of four nodes at a time where the registers allow it
+        // z series of four nodes at a time above npw 32: 8% faster there though
+        // it adds spills; below, where a node's products are half as long, the
+        // spills cost 5%
         constexpr int ZB = NB >= 3 ? 4 : 1;
         double2 zb[ZB];
         for (int c = 0; c < half; ++c) {
@@ -2708,9 +2714,72 @@ void launch_top_leaves(const TopLeafArgs& a, hipStream_t s)
 }
 
 // ---------------------------------------------------------------------------
+// Source staging of the near field (k_direct3, 256 threads): the sources of a
+// unit's source boxes lie in many short ranges (a leaf holds a few to 100), so
+// up to 64 ranges are scanned at once and their sources staged 256 at a time,
+// whichever boxes they come from -- two dependent loads and two barriers per
+// 256 sources instead of per box.  Every wavefront scans the ranges for itself:
+// no barrier, and a unit of one box pays nothing.  In 2D, with at most 13 boxes
+// to a list, a stage per box is the faster: 38 against 46 us on 10^5 mixture
+// points.
+// ---------------------------------------------------------------------------
+constexpr int NEAR_RANGES = 64;
+struct NearBatch {          // a wavefront's own copy
+    int off[NEAR_RANGES];   // first staged position of every range
+    int st[NEAR_RANGES];    // its first source
+};
+
+// ranges list[b0 .. b0 + n), n <= NEAR_RANGES; returns the number of their
+// sources
+__device__ __forceinline__ int near_ranges(NearBatch& B, const int* list, const int2* se, int b0,
+                                           int n)
+{
+    const int lane = threadIdx.x & 63;
+    int c = 0, s = 0;
+    if (lane < n) {
+        const int2 r = se[list[b0 + lane]];
+        s = r.x;
+        c = max(r.y - r.x, 0);
+    }
+    int x = c;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o);
+        if (lane >= o) x += y;
+    }
+    // a wavefront's LDS accesses keep their order; the fences hold the compiler
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    B.off[lane] = x - c;
+    B.st[lane] = s;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    return __shfl(x, 63);
+}
+
+// the source at staged position p of a batch of n ranges
+__device__ __forceinline__ int near_source(const NearBatch& B, int n, int p)
+{
+    int lo = 0, hi = n - 1;  // the last range that starts at or before p
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (B.off[mid] <= p) lo = mid; else hi = mid - 1;
+    }
+    return B.st[lo] + p - B.off[lo];
+}
+
+// threads per target (neighbouring lanes, a power of two, at most 64) when
+// 256 threads take cnt <= 256 targets
+__device__ __forceinline__ int near_split(int cnt)
+{
+    int k = 1;
+    while (k < 64 && 2 * k * cnt <= 256) k *= 2;
+    return k;
+}
+
+// ---------------------------------------------------------------------------
 // Step 6, near field (g3d_directcp/cg/ch_vec g3ddirect.f:3-206 called from
 // fgt3d.f:1460-1512): one block per target unit, the sources of its source
-// boxes staged in LDS 256 at a time (near_stage.hpp), up to 64 lanes a target
+// boxes staged in LDS 256 at a time, up to 64 lanes a target
 // where a unit has few; pairs with r^2 < dmax; accumulated.  Bound by the
 // latency of the staging.  Against a stage per source box: 2053 uniform points,
 // delta 1e-3 (up to 27 boxes of 20 sources a unit) 87 -> 25 us, 8M shell
